@@ -252,26 +252,12 @@ __global__ void k_batch_zero_norms(double* norms, const int* active, int n) {
 }
 
 // ---------------------------------------------------------------------------
-// bottom of every problem: relax(m_bottom) from zero, then BiCGStabSolver::solve
+// The general bottom kernel, for levels whose slot tables do not apply (bottom.hip): relax(m_bottom) from zero, then BiCGStabSolver::solve
 // (BiCGStabSolver.H:199-519) in FP64 on the deepest level, one workgroup per problem.
 // Level operations mirror AMRPoissonOp on that level (homogeneous BC) and the
 // reductions keep the reference orders (dot: per box serially in Fortran order,
 // boxes in layout order; norm 2: FArrayBox::sumPow column sums per box).
 // ---------------------------------------------------------------------------
-struct BottomArgs {
-  int imax;
-  double reps, hang, small;
-  int numRestarts;
-  int nbottom;                 // relax iterations before the Krylov solve
-  int relaxFirst;              // 1: zero the correction and relax nbottom times first (the
-                               // whole bottom of MultiGrid::cycle); 0: start from the correction
-  int ldsDoubles;              // dynamic LDS of the launch, in doubles: a problem whose ten
-                               // Krylov vectors fit keeps them there instead of in scratch
-};
-// dynamic LDS offered to a single solver's bottom Krylov vectors (the static LDS of
-// the kernel is at most 70 KB, the workgroup may hold 160 KB)
-constexpr int kBottomLdsDoubles = 8192;
-
 // A walk over the cells of a box of extents (ea, eb, *), a fastest, in steps of
 // `step` cells: the position (a, b, c) and its element offset are advanced with
 // adds and compares only (no division per cell).
@@ -615,16 +601,16 @@ constexpr int kStage = kFillSteps * kBottomThreads + kBottomThreads;
 constexpr int kUS = 4, kUE = 8;      // cells per thread and pass: stencil / elementwise sweeps
 template <class T, bool TREE>
 __global__ void __launch_bounds__(kBottomThreads)
-    k_batch_bottom(const BatchBottom* __restrict__ bots, const BatchCoef* __restrict__ bcoef,
-                   const DBox* __restrict__ bboxes, T* const* __restrict__ corr, const T* const* __restrict__ res,
-                   double* __restrict__ scratch, const long long* __restrict__ soff, const double* __restrict__ metric,
-                   const int* __restrict__ active, int* __restrict__ stats, BottomArgs ba) {
+    k_batch_bottom(const BatchBottom* __restrict__ bots, const DBox* __restrict__ bboxes,
+                   const long long* __restrict__ soff, BottomLaunch<T> A) {
   // cells per thread and pass of the stencil / elementwise sweeps (fewer cells per
   // pass, for more problems per CU, measured slower: the sweeps are bound by the
   // loads each thread keeps in flight)
   constexpr int US = kUS, UE = kUE;
   const int p = blockIdx.x;
-  if (!active[p]) return;
+  if (A.active && !A.active[p]) return;
+  if (A.plans && A.plans[p].nslot) return;  // k_bottom's problem
+  const BottomParams& ba = A.par;
   __shared__ double sh[kBottomThreads];
   __shared__ double stage[kStage];
   __shared__ DBox sbox[kBoxCache];
@@ -634,7 +620,7 @@ __global__ void __launch_bounds__(kBottomThreads)
   const int tid = threadIdx.x;
   // fields are addressed from the base of the level's ghosted rectangle
   BottomLevel L;
-  L.cf = bcoef[p];
+  L.cf = A.coef ? A.coef[p] : A.cf;
   L.R = bt.rect;
   L.R.off = 0;
   L.tid = tid;
@@ -667,8 +653,8 @@ __global__ void __launch_bounds__(kBottomThreads)
   B.maxCol = smax[1];
   B.ncol = 0;
   for (int q = 0; q < B.n; q++) B.ncol += B.get(q).hi[0] - B.get(q).lo[0] + 1;
-  T* e32 = corr[p] + bt.rect.off;
-  const T* r32 = res[p] + bt.rect.off;
+  T* e32 = (A.corr ? A.corr[p] : A.corr1) + bt.rect.off;
+  const T* r32 = (A.res ? A.res[p] : A.res1) + bt.rect.off;
   if (ba.relaxFirst) {
     // MultiGrid::cycle at the bottom: the correction is zero on entry
     L.sweep<UE>([&](int) { return 0; }, [&](int c, int, int, int, int) { e32[c] = T(0.0); });
@@ -676,11 +662,7 @@ __global__ void __launch_bounds__(kBottomThreads)
     if (L.ncell == 1) return;  // m_bottomCells == 1: relax only
   }
   const long long vs = 15 + (long long)L.R.sz * (L.nz + 2);  // elements per scratch vector
-  // the ten vectors live in LDS when they fit there (every cell a vector is read at
-  // is written first in the solve, and its ghost cells are never used: the face
-  // rules replace them), else in the problem's global scratch
-  extern __shared__ double ldsVec[];
-  double* base = (10 * vs <= ba.ldsDoubles) ? ldsVec + 15 : scratch + soff[p] + 15;  // rectangle base of the first
+  double* base = A.vecs + soff[p] + 15;  // rectangle base of the first
   double *x = base, *b = base + vs, *r = base + 2 * vs, *r_tilde = base + 3 * vs, *e = base + 4 * vs,
          *pp = base + 5 * vs, *p_tilde = base + 6 * vs, *s_tilde = base + 7 * vs, *t = base + 8 * vs,
          *v = base + 9 * vs;
@@ -813,8 +795,8 @@ __global__ void __launch_bounds__(kBottomThreads)
     else return norm(a);
   };
 
-  const double eps = metric[2 * p + 1];
-  const double convergenceMetric = metric[2 * p];
+  const double eps = A.metric ? A.metric[2 * p + 1] : A.eps1;
+  const double convergenceMetric = A.metric ? A.metric[2 * p] : A.metric1;
   int recount = 0;
   residual(r, x, b);  // setToZero(r) then residual: every valid cell is written
   assign(r_tilde, r);
@@ -907,7 +889,7 @@ __global__ void __launch_bounds__(kBottomThreads)
     }
   }
   if (!done) incr(x, e, 1.0);
-  if (tid == 0) stats[p] += iter;
+  if (tid == 0 && A.stats) A.stats[p] += iter;
   // round the correction back into the V-cycle's precision
   L.sweep<UE>([&](int c) { return x[c]; }, [&](int c, int, int, int, double w) { e32[c] = (T)w; });
 }
@@ -1062,6 +1044,8 @@ BatchSolver::BatchSolver(Context* ctx, std::vector<BatchProblemSpec> problems, i
   std::vector<BatchCoef> bcoef;
   std::vector<void*> corrp, resp;
   long long soff = 0;
+  std::vector<BottomTables> tabs(m_np);
+  std::vector<BottomTables*> tabp;
   for (int p = 0; p < m_np; p++) {
     const int db = m_ndepth[p] - 1;
     const Depth& L = m_depth[db];
@@ -1091,11 +1075,34 @@ BatchSolver::BatchSolver(Context* ctx, std::vector<BatchProblemSpec> problems, i
     corrp.push_back(L.corr);
     resp.push_back(L.res);
     (void)es;
-    // scratch: 10 FP64 vectors of the same ghosted shape, each addressed with the
-    // bottom rectangle's own offsets
-    const long long vs = 15 + (long long)b.rect.sz * (b.rect.hi[2] - b.rect.lo[2] + 3);
+    // the slot tables where they apply, else scratch for the general kernel: 10 FP64 vectors
+    // of the same ghosted shape, each addressed with the bottom rectangle's own offsets
+    BottomTables& t = tabs[p];
+    tabp.push_back(&t);
+    const DBox& R = b.rect;
+    const Box rb(IV{R.lo[0], R.lo[1], R.lo[2]}, IV{R.hi[0], R.hi[1], R.hi[2]});
+    const bool slots = t.build(g.boxes, rb, L.h_coef[p].kind, 1, 0, [&](int, int i, int j, int k) {
+      return (i - R.lo[0] + 1) + (long long)(j - R.lo[1] + 1) * R.sy + (long long)(k - R.lo[2] + 1) * R.sz;
+    });
     h_bscratchOff.push_back(soff);
-    soff += 10 * vs;
+    if (slots) {
+      t.plan.base = R.off;
+      t.plan.vec = soff / 2;
+      soff += 2 * t.pairs();
+      m_bslots = std::max(m_bslots, t.plan.nslot);
+      m_blds = std::max(m_blds, t.ldsBytes());
+    } else {
+      t.plan = BottomPlan{};
+      m_bgeneral++;
+      soff += 10 * (15 + (long long)b.rect.sz * (b.rect.hi[2] - b.rect.lo[2] + 3));
+      soff += soff & 1;
+    }
+  }
+  d_btab = BottomTables::upload(m_ctx, tabp, &m_bytes);
+  {
+    std::vector<BottomPlan> plans;
+    for (auto& t : tabs) plans.push_back(t.plan);
+    d_bplan = upload(m_ctx, plans, &m_bytes);
   }
   d_bottom = upload(m_ctx, h_bottom, &m_bytes);
   d_bbox = upload(m_ctx, h_bbox, &m_bytes);
@@ -1120,7 +1127,7 @@ BatchSolver::~BatchSolver() {
     f(L.d_rect); f(L.d_coef); f(L.d_tiles); f(L.d_ctiles); f(L.d_items); f(L.d_wStart); f(L.corr); f(L.res); f(L.tmp);
   }
   f(m_phi); f(m_rhs); f(m_norm); f(d_active); f(d_metric); f(d_bstats); f(d_bottom); f(d_bbox); f(m_bcoef);
-  f(d_corrPtr); f(d_resPtr); f(d_bscratchOff); f(d_bscratch);
+  f(d_corrPtr); f(d_resPtr); f(d_bscratchOff); f(d_bscratch); f(d_btab); f(d_bplan);
   if (h_norm) (void)hipHostFree(h_norm);
 }
 
@@ -1343,15 +1350,23 @@ void BatchSolver::vcycle() {
     BATCH_LAUNCH(k_batch_restrict<T>, C.tileStart[np], 256, C.d_tiles, 6, 2, C.d_rect, F.d_rect, F.d_coef, d_active,
                  (T*)C.res, (const T*)F.corr, (const T*)F.res);
   }
-  // Krylov vectors in global scratch: a batch's bottom time is set by its largest
-  // bottoms, which do not fit in LDS (measured no faster with the small ones there)
-  BottomArgs ba{80, 1e-12, 1e-8, 1e-30, 5, m_nbottom, 1, 0};
-  if (m_treeOrder)
-    BATCH_LAUNCH((k_batch_bottom<T, true>), m_np, kBottomThreads, d_bottom, m_bcoef, d_bbox, (T* const*)d_corrPtr,
-                 (const T* const*)d_resPtr, d_bscratch, d_bscratchOff, d_metric, d_active, d_bstats, ba);
-  else
-    BATCH_LAUNCH((k_batch_bottom<T, false>), m_np, kBottomThreads, d_bottom, m_bcoef, d_bbox, (T* const*)d_corrPtr,
-                 (const T* const*)d_resPtr, d_bscratch, d_bscratchOff, d_metric, d_active, d_bstats, ba);
+  BottomLaunch<T> bl;
+  bl.plans = (const BottomPlan*)d_bplan;
+  bl.coef = m_bcoef;
+  bl.corr = (T* const*)d_corrPtr;
+  bl.res = (const T* const*)d_resPtr;
+  bl.vecs = d_bscratch;
+  bl.metric = d_metric;
+  bl.active = d_active;
+  bl.stats = d_bstats;
+  bl.par = BottomParams{80, 1e-12, 1e-8, 1e-30, 5, m_nbottom, 1};
+  if (m_bslots > 0) launch_bottom<T>(m_ctx, bl, m_np, m_bslots, m_blds, m_treeOrder);
+  if (m_bgeneral > 0) {
+    if (m_treeOrder)
+      BATCH_LAUNCH((k_batch_bottom<T, true>), m_np, kBottomThreads, d_bottom, d_bbox, d_bscratchOff, bl);
+    else
+      BATCH_LAUNCH((k_batch_bottom<T, false>), m_np, kBottomThreads, d_bottom, d_bbox, d_bscratchOff, bl);
+  }
   for (int d = D - 2; d >= 0; d--) {
     const int np = m_depth[d + 1].np;
     Depth& F = m_depth[d];
@@ -1562,7 +1577,7 @@ std::vector<double> BatchSolver::tuneRelax() {
 
 // ---------------------------------------------------------------------------
 // DeviceBottomSolver: the bottom BiCGStab of one hierarchy's multigrid as one
-// workgroup on the device (the batched bottom kernel on a one-entry table)
+// workgroup on the device
 // ---------------------------------------------------------------------------
 template <class T>
 DeviceBottomSolver<T>::~DeviceBottomSolver() {
@@ -1572,17 +1587,17 @@ template <class T>
 void DeviceBottomSolver<T>::release() {
   if (m_ctx->dry) return;
   if (m_ctx->stream) (void)hipStreamSynchronize(m_ctx->stream);
-  void* ps[] = {d_bottom, d_bcoef, d_bbox, d_ptrs, d_scratch, d_soff, d_metric, d_active, d_stats};
+  void* ps[] = {d_bottom, d_bbox, d_soff, d_scratch, d_stats, d_tab, d_plan};
   for (void* p : ps)
     if (p) (void)hipFree(p);
-  if (h_stage) (void)hipHostFree(h_stage);
-  d_bottom = nullptr; d_bcoef = nullptr; d_bbox = nullptr; d_ptrs = nullptr; d_scratch = nullptr;
-  d_soff = nullptr; d_metric = nullptr; d_active = nullptr; d_stats = nullptr; h_stage = nullptr;
+  d_bottom = nullptr; d_bbox = nullptr; d_soff = nullptr; d_scratch = nullptr; d_stats = nullptr;
+  d_tab = nullptr; d_plan = nullptr;
+  m_nc = 0;
 }
-// the operator's coefficients as the bottom kernel reads them (face rules are set by define)
+// the operator's coefficients as the bottom kernels read them (face rules are set by define)
 template <class T>
-static BatchCoef bottom_coef(const AMRPoissonOp<T>* ap) {
-  BatchCoef c{};
+static BatchCoef bottom_coef(const AMRPoissonOp<T>* ap, const BatchCoef& faces) {
+  BatchCoef c = faces;
   c.dx = ap->m_dx;
   c.dxinv = 1.0 / (c.dx * c.dx);
   double sum_b = 0.0;
@@ -1594,128 +1609,156 @@ static BatchCoef bottom_coef(const AMRPoissonOp<T>* ap) {
   return c;
 }
 template <class T>
+bool DeviceBottomSolver<T>::buildSlots(int nc) {
+  const DeviceLayout& L = *m_lay;
+  long long n = 0;
+  m_nc = 0;
+  if (d_tab || d_plan || d_scratch) {
+    (void)hipStreamSynchronize(m_ctx->stream);
+    for (void* p : {d_tab, d_plan, (void*)d_scratch})
+      if (p) (void)hipFree(p);
+    d_tab = d_plan = nullptr;
+    d_scratch = nullptr;
+  }
+  const long long cs = nc > 1 ? LevelData<T>::compStride(&L) : L.slab;
+  if (!m_tab.build(L.dbl.boxes, L.rect, m_coef.kind, nc, cs, [&](int b, int i, int j, int k) { return L.index(b, i, j, k); }))
+    return false;
+  d_tab = BottomTables::upload(m_ctx, {&m_tab}, &n);
+  d_plan = upload(m_ctx, std::vector<BottomPlan>{m_tab.plan}, &n);
+  hip_check(hipMalloc(&d_scratch, 16 * (size_t)m_tab.pairs()), "hipMalloc bottom vectors");
+  m_nc = nc;
+  return true;
+}
+template <class T>
 void DeviceBottomSolver<T>::define(LinearOp<LevelData<T>>* op, bool homogeneous) {
   m_fallback.define(op, homogeneous);
   auto* ap = dynamic_cast<AMRPoissonOp<T>*>(op);
   // variable coefficients or Jacobi relaxation: the host-driven solve
   const bool vc = ap && (ap->m_vc || ap->m_relaxMode != 1);
-  if (m_device && op == m_boundOp && homogeneous && !vc) return;  // MultiGrid re-binds its bottom at every solve
-  m_device = false;
+  if (m_mode != HOST && op == m_boundOp && homogeneous && !vc) return;  // MultiGrid re-binds its bottom at every solve
+  m_mode = HOST;
   m_boundOp = op;
-  if (!homogeneous || !ap || vc || !ap->m_lay->merged || m_ctx->dry) return;
+  if (!homogeneous || !ap || vc || m_ctx->dry) return;
   release();
   const DeviceLayout& L = *ap->m_lay;
   m_lay = &L;
-  BatchBottom b{};
-  b.rect = L.h_boxes[L.nbox];
-  b.cells = L.valid_cells;
-  b.box0 = 0;
-  b.nbox = L.nbox;
-  // one thread per reduction chain (two dot products share a pass; a norm has a
-  // chain per box column): otherwise the host-driven solve
-  if (2 * b.nbox > kBottomThreads) return;
-  long long widths = 0;
-  for (int q = 0; q < L.nbox; q++) widths += L.h_boxes[q].hi[0] - L.h_boxes[q].lo[0] + 1;
-  if (widths > kBottomThreads) return;
-  std::vector<DBox> boxes;
-  for (int q = 0; q < L.nbox; q++) {
-    const DBox& x0 = L.h_boxes[q];
-    DBox x = x0;  // addressed in the scratch vectors (rectangle at offset 15)
-    x.off = (x0.lo[0] - b.rect.lo[0]) + (long long)(x0.lo[1] - b.rect.lo[1]) * b.rect.sy +
-            (long long)(x0.lo[2] - b.rect.lo[2]) * b.rect.sz;
-    boxes.push_back(x);
-  }
-  BatchCoef c = bottom_coef(ap);
-  // the bottom of a merged multigrid level is a whole (coarsened) domain: every
-  // face is a domain face with the operator's BC type
+  m_ap = ap;
+  // the level covers its whole domain (a level with coarse-fine faces keeps the host-driven
+  // solver), so every face is a domain face with the operator's BC type
+  if (!(L.rect == ap->m_domain) || L.valid_cells != L.rect.npts()) return;
+  m_coef = BatchCoef{};
   for (int dir = 0; dir < 3; dir++)
     for (int side = 0; side < 2; side++) {
-      const int face = side ? b.rect.hi[dir] : b.rect.lo[dir];
-      const int dface = side ? ap->m_domain.hi[dir] : ap->m_domain.lo[dir];
-      if (face != dface) return;  // a level with coarse-fine faces keeps the host-driven solver
-      if (ap->m_bc.type[side][dir] > 1) return;  // quadratic Dirichlet faces: the host-driven solver
-      c.kind[dir][side] = ap->m_bc.type[side][dir];
-      c.val[dir][side] = ap->m_bc.val[side][dir];
+      if (ap->m_bc.type[side][dir] == 2) return;  // quadratic Dirichlet faces: the host-driven solver
+      m_coef.kind[dir][side] = ap->m_bc.type[side][dir];
+      m_coef.val[dir][side] = ap->m_bc.val[side][dir];
     }
-  const long long vs = 15 + (long long)b.rect.sz * (b.rect.hi[2] - b.rect.lo[2] + 3);
-  m_vs = vs;
-  m_ap = ap;
-  m_coef = c;
   long long bytes = 0;
-  d_bottom = upload(m_ctx, std::vector<BatchBottom>{b}, &bytes);
-  d_bcoef = upload(m_ctx, std::vector<BatchCoef>{c}, &bytes);
-  d_bbox = upload(m_ctx, boxes, &bytes);
-  d_soff = upload(m_ctx, std::vector<long long>{0}, &bytes);
-  d_active = upload(m_ctx, std::vector<int>{1}, &bytes);
+  if (buildSlots(ap->m_ncomp)) {
+    m_mode = SLOTS;
+  } else {
+    for (int dir = 0; dir < 3; dir++)
+      if (m_coef.kind[dir][0] == 3) return;
+    if (!L.merged) return;
+    BatchBottom b{};
+    b.rect = L.h_boxes[L.nbox];
+    b.cells = L.valid_cells;
+    b.box0 = 0;
+    b.nbox = L.nbox;
+    // one thread per reduction chain (two dot products share a pass; a norm has a
+    // chain per box column): otherwise the host-driven solve
+    if (2 * b.nbox > kBottomThreads) return;
+    long long widths = 0;
+    for (int q = 0; q < L.nbox; q++) widths += L.h_boxes[q].hi[0] - L.h_boxes[q].lo[0] + 1;
+    if (widths > kBottomThreads) return;
+    std::vector<DBox> boxes;
+    for (int q = 0; q < L.nbox; q++) {
+      const DBox& x0 = L.h_boxes[q];
+      DBox x = x0;  // addressed in the scratch vectors (rectangle at offset 15)
+      x.off = (x0.lo[0] - b.rect.lo[0]) + (long long)(x0.lo[1] - b.rect.lo[1]) * b.rect.sy +
+              (long long)(x0.lo[2] - b.rect.lo[2]) * b.rect.sz;
+      boxes.push_back(x);
+    }
+    m_vs = 15 + (long long)b.rect.sz * (b.rect.hi[2] - b.rect.lo[2] + 3);
+    d_bottom = upload(m_ctx, std::vector<BatchBottom>{b}, &bytes);
+    d_bbox = upload(m_ctx, boxes, &bytes);
+    d_soff = upload(m_ctx, std::vector<long long>{0}, &bytes);
+    hip_check(hipMalloc(&d_scratch, sizeof(double) * 10 * m_vs), "hipMalloc bottom scratch");
+    m_mode = GENERAL;
+  }
   d_stats = upload(m_ctx, std::vector<int>{0}, &bytes);
-  hip_check(hipMalloc(&d_scratch, sizeof(double) * 10 * vs), "hipMalloc bottom scratch");
-  hip_check(hipMalloc(&d_metric, sizeof(double) * 2), "hipMalloc bottom metric");
-  hip_check(hipMalloc(&d_ptrs, sizeof(void*) * 2), "hipMalloc bottom pointers");
-  hip_check(hipHostMalloc(&h_stage, 64 + sizeof(BatchCoef)), "hipHostMalloc bottom staging");
-  m_device = true;
-  setConvergenceMetrics(m_metric, m_eps);
 }
 template <class T>
 void DeviceBottomSolver<T>::setConvergenceMetrics(double metric, double tol) {
   m_metric = metric;
   m_eps = tol;
   m_fallback.setConvergenceMetrics(metric, tol);
-  if (!m_device) return;
-  double* h = (double*)h_stage;
-  (void)hipStreamSynchronize(m_ctx->stream);  // the staging buffer may still feed an earlier copy
-  h[0] = metric;
-  h[1] = tol;
-  hip_check(hipMemcpyAsync(d_metric, h, sizeof(double) * 2, hipMemcpyHostToDevice, m_ctx->stream), "bottom metric");
+}
+template <class T>
+bool DeviceBottomSolver<T>::checkBound() const {
+  return !m_ap->m_vc && m_ap->m_relaxMode == 1;
+}
+// The fields' buffers move (the relaxation swaps them) and the coefficients may be reset
+// between solves, so both go with each launch: no copy, no wait.
+template <class T>
+void DeviceBottomSolver<T>::launchSlots(LevelData<T>& phi, const LevelData<T>& rhs, int nrelax, bool relaxFirst) {
+  if (phi.lay != m_lay || rhs.lay != m_lay || rhs.nc != phi.nc)
+    throw std::runtime_error("DeviceBottomSolver: layout mismatch");
+  BottomLaunch<T> a;
+  a.plans = (const BottomPlan*)d_plan;
+  a.cf = bottom_coef(m_ap, m_coef);
+  a.corr1 = phi.d;
+  a.res1 = rhs.d;
+  a.vecs = d_scratch;
+  a.metric1 = m_metric;
+  a.eps1 = m_eps;
+  a.stats = d_stats;
+  a.par = BottomParams{m_fallback.m_imax, m_fallback.m_reps, m_fallback.m_hang, m_fallback.m_small,
+                       m_fallback.m_numRestarts, nrelax, relaxFirst ? 1 : 0};
+  launch_bottom<T>(m_ctx, a, 1, m_tab.plan.nslot, m_tab.ldsBytes(), false);
+}
+template <class T>
+bool DeviceBottomSolver<T>::relaxSolveFromZero(LevelData<T>& phi, const LevelData<T>& rhs, int nrelax) {
+  // (the event profiler counts the relaxation's launches: they stay apart while it is on)
+  if (m_mode != SLOTS || phi.nc != m_nc || m_lay->valid_cells == 1 || !checkBound() || m_ctx->prof) return false;
+  launchSlots(phi, rhs, nrelax, true);
+  return true;
 }
 template <class T>
 void DeviceBottomSolver<T>::solve(LevelData<T>& phi, const LevelData<T>& rhs) {
-  if (m_device && (static_cast<const AMRPoissonOp<T>*>(m_ap)->m_vc ||
-                   static_cast<const AMRPoissonOp<T>*>(m_ap)->m_relaxMode != 1))
-    throw std::runtime_error("DeviceBottomSolver: operator changed after define");
-  if (!m_device || phi.nc > 1) {  // fields of several components: the host-driven solve
+  if (m_mode != HOST && !checkBound()) throw std::runtime_error("DeviceBottomSolver: operator changed after define");
+  if (m_mode == SLOTS && phi.nc == m_nc) {
+    launchSlots(phi, rhs, 0, false);
+    return;
+  }
+  if (m_mode != GENERAL || phi.nc > 1) {
     m_fallback.solve(phi, rhs);
     return;
   }
   if (phi.lay != m_lay || rhs.lay != m_lay) throw std::runtime_error("DeviceBottomSolver: layout mismatch");
-  // the fields' buffers move (the relaxation swaps them), so their addresses go with
-  // each launch; the operator's coefficients may have been reset since define
-  void** h = (void**)((char*)h_stage + 32);
-  (void)hipStreamSynchronize(m_ctx->stream);
-  h[0] = phi.d;
-  h[1] = (void*)rhs.d;
-  hip_check(hipMemcpyAsync(d_ptrs, h, sizeof(void*) * 2, hipMemcpyHostToDevice, m_ctx->stream), "bottom pointers");
-  const auto* ap = static_cast<const AMRPoissonOp<T>*>(m_ap);
-  if (ap->m_alpha != m_coef.alpha || ap->m_beta != m_coef.beta || ap->m_dx != m_coef.dx) {
-    BatchCoef c = bottom_coef(ap);
-    for (int dir = 0; dir < 3; dir++)
-      for (int side = 0; side < 2; side++) {
-        c.kind[dir][side] = m_coef.kind[dir][side];
-        c.val[dir][side] = m_coef.val[dir][side];
-      }
-    m_coef = c;
-    std::memcpy((char*)h_stage + 64, &m_coef, sizeof(BatchCoef));
-    hip_check(hipMemcpyAsync(d_bcoef, (char*)h_stage + 64, sizeof(BatchCoef), hipMemcpyHostToDevice, m_ctx->stream),
-              "bottom coefficients");
-  }
-  // the Krylov vectors in LDS when the level is small enough
-  const int lds = (10 * m_vs <= kBottomLdsDoubles) ? (int)(10 * m_vs) : 0;
-  BottomArgs ba{m_fallback.m_imax, m_fallback.m_reps, m_fallback.m_hang, m_fallback.m_small,
-                m_fallback.m_numRestarts, 0, 0, lds};
-  hipLaunchKernelGGL((k_batch_bottom<T, false>), dim3(1), dim3(kBottomThreads), sizeof(double) * lds, m_ctx->stream,
-                     (const BatchBottom*)d_bottom,
-                     (const BatchCoef*)d_bcoef, (const DBox*)d_bbox, (T* const*)d_ptrs,
-                     (const T* const*)((void**)d_ptrs + 1), d_scratch, (const long long*)d_soff,
-                     (const double*)d_metric, (const int*)d_active, (int*)d_stats, ba);
+  BottomLaunch<T> a;
+  a.cf = bottom_coef(m_ap, m_coef);
+  a.corr1 = phi.d;
+  a.res1 = rhs.d;
+  a.vecs = d_scratch;
+  a.metric1 = m_metric;
+  a.eps1 = m_eps;
+  a.stats = d_stats;
+  a.par = BottomParams{m_fallback.m_imax, m_fallback.m_reps, m_fallback.m_hang, m_fallback.m_small,
+                       m_fallback.m_numRestarts, 0, 0};
+  hipLaunchKernelGGL((k_batch_bottom<T, false>), dim3(1), dim3(kBottomThreads), 0, m_ctx->stream,
+                     (const BatchBottom*)d_bottom, (const DBox*)d_bbox, (const long long*)d_soff, a);
   hip_check(hipGetLastError(), "k_batch_bottom");
 }
 template <class T>
 long long DeviceBottomSolver<T>::totalIterations() {
-  if (!m_device) return m_fallback.m_total_iters;
+  if (m_mode == HOST) return m_fallback.m_total_iters;
   int v = 0;
-  hip_check(hipMemcpyAsync(h_stage, d_stats, sizeof(int), hipMemcpyDeviceToHost, m_ctx->stream), "bottom stats");
+  hip_check(hipMemcpyAsync(m_ctx->h_scalars + 63, d_stats, sizeof(int), hipMemcpyDeviceToHost, m_ctx->stream),
+            "bottom stats");
   m_ctx->sync();
-  std::memcpy(&v, h_stage, sizeof(int));
-  return v;
+  std::memcpy(&v, m_ctx->h_scalars + 63, sizeof(int));
+  return v + m_fallback.m_total_iters;
 }
 template class DeviceBottomSolver<double>;
 template class DeviceBottomSolver<float>;

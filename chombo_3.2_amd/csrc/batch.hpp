@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "amrpoissonop.hpp"
+#include "bottom.hpp"
 #include "fused.hpp"
 #include "ops.hpp"
 #include "plans.hpp"
@@ -32,14 +33,6 @@ struct BatchProblemSpec {
   DBL boxes;                  // its DisjointBoxLayout (fixes the multigrid depth and the bottom boxes)
   double dx = 1, alpha = 0, beta = 1;
   BCSpec bc{};
-};
-
-// per problem and depth: the operator's coefficients and face rules
-struct BatchCoef {
-  double dxinv, lambda, alpha, beta, dx;
-  int lap;          // 1: GSRBLAPLACIAN / OPERATORLAP forms (alpha == 0 and beta == 1)
-  int kind[3][2];   // face rule: 0 Neumann, 1 Dirichlet
-  double val[3][2]; // face values (outer residual only; every other use is homogeneous)
 };
 
 // the bottom of one problem: its level and boxes at its deepest depth
@@ -54,8 +47,10 @@ struct BatchBottom {
 // deepest level, homogeneous) run on the device as one workgroup: the control flow,
 // level operations and reduction orders of BiCGStabSolver, with no host round
 // trip per iteration.  With T = float it widens the correction and the residual
-// and solves in FP64, as PromotedBottomSolver does.  Levels that are not stored
-// merged over a whole domain use the host-driven BiCGStabSolver (FP64 only).
+// and solves in FP64, as PromotedBottomSolver does.  It takes levels of constant
+// coefficients over a whole domain, merged or per box, of any component count
+// (bottom.hip; levels too large for that kernel: the general kernel of batch.hip, merged
+// levels of one component only).  Others use the host-driven BiCGStabSolver.
 template <class T>
 class DeviceBottomSolver : public LinearSolver<LevelData<T>> {
  public:
@@ -65,23 +60,33 @@ class DeviceBottomSolver : public LinearSolver<LevelData<T>> {
   DeviceBottomSolver& operator=(const DeviceBottomSolver&) = delete;
   void define(LinearOp<LevelData<T>>* op, bool homogeneous) override;
   void solve(LevelData<T>& phi, const LevelData<T>& rhs) override;
+  bool relaxSolveFromZero(LevelData<T>& phi, const LevelData<T>& rhs, int nrelax) override;
   void setConvergenceMetrics(double metric, double tol) override;
   long long totalIterations();
-  bool onDevice() const { return m_device; }
+  bool onDevice() const { return m_mode != HOST; }
   BiCGStabSolver<LevelData<T>> m_fallback;   // parameters (m_imax, m_reps, ...) are read from here
 
  private:
+  enum Mode { HOST, GENERAL, SLOTS };
   Context* m_ctx;
-  bool m_device = false;
+  Mode m_mode = HOST;
   const DeviceLayout* m_lay = nullptr;
   const void* m_boundOp = nullptr;
-  const void* m_ap = nullptr;     // the bound AMRPoissonOp<T>
-  BatchCoef m_coef{};             // coefficients uploaded for it
-  long long m_vs = 0;             // elements per Krylov vector of the bound level
+  const AMRPoissonOp<T>* m_ap = nullptr;
+  BatchCoef m_coef{};             // face rules of the bound level (its coefficients are taken at each solve)
   double m_metric = -1.0, m_eps = 1e-6;
-  void *d_bottom = nullptr, *d_bcoef = nullptr, *d_bbox = nullptr, *d_ptrs = nullptr, *d_soff = nullptr;
-  void *d_active = nullptr, *d_stats = nullptr, *h_stage = nullptr;
-  double *d_scratch = nullptr, *d_metric = nullptr;
+  int* d_stats = nullptr;
+  double* d_scratch = nullptr;    // Krylov vectors
+  // SLOTS
+  BottomTables m_tab;
+  void *d_tab = nullptr, *d_plan = nullptr;
+  int m_nc = 0;                   // components the tables are for
+  bool buildSlots(int nc);
+  void launchSlots(LevelData<T>& phi, const LevelData<T>& rhs, int nrelax, bool relaxFirst);
+  // GENERAL
+  long long m_vs = 0;             // elements per Krylov vector
+  void *d_bottom = nullptr, *d_bbox = nullptr, *d_soff = nullptr;
+  bool checkBound() const;        // the operator still has the form it was bound with
   void release();
 };
 
@@ -181,7 +186,10 @@ class BatchSolver {
   void** d_resPtr = nullptr;
   std::vector<DBox> h_bbox;                      // bottom boxes (addresses in each bottom's merged array)
   DBox* d_bbox = nullptr;
-  double* d_bscratch = nullptr;                  // 10 FP64 vectors per problem (bottom BiCGStab)
+  double* d_bscratch = nullptr;                  // bottom BiCGStab vectors of every problem
+  void *d_btab = nullptr, *d_bplan = nullptr;    // slot tables and plans (bottom.hip), per slot
+  int m_bslots = 0, m_bgeneral = 0;              // largest plan; problems without one (general kernel)
+  size_t m_blds = 0;
   std::vector<long long> h_bscratchOff;
   long long* d_bscratchOff = nullptr;
   double* d_metric = nullptr;                    // per slot: convergence metric and eps of the bottom solve

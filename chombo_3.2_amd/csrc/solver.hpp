@@ -79,6 +79,12 @@ class LinearSolver {
   virtual ~LinearSolver() {}
   virtual void define(LinearOp<T>* op, bool homogeneous) = 0;
   virtual void solve(T& phi, const T& rhs) = 0;
+  // setToZero(phi), the operator's relax(phi, rhs, nrelax) and solve(phi, rhs) in one step;
+  // false (nothing done) where the solver has no such step
+  virtual bool relaxSolveFromZero(T& phi, const T& rhs, int nrelax) {
+    (void)phi; (void)rhs; (void)nrelax;
+    return false;
+  }
   virtual void setConvergenceMetrics(double metric, double tolerance) = 0;
 };
 
@@ -256,7 +262,7 @@ class MultiGrid {
     if (depth == m_depth - 1) {
       if (m_bottomCells == 1) {
         relax(1);
-      } else {
+      } else if (!zero || !m_bottomSolver->relaxSolveFromZero(correction, residual, m_bottom)) {
         relax(m_bottom);
         m_bottomSolver->solve(correction, residual);
       }
