@@ -213,23 +213,25 @@ void AMRPoissonOp<Real>::incrFromZero(T& lhs, const T& x) {
   ops::incr_from_zero<Real>(*lhs.lay, lhs.d, x.d);
 }
 template <class Real>
-void AMRPoissonOp<Real>::incrAssignUpdate(T& m, T& d, T& phi) {
+void AMRPoissonOp<Real>::correctUpdate(T& m, const T& d, LevelData<double>& phi, bool storeM) {
   if (m.nc > 1) {
     for (int c = 0; c < m.nc; c++) {
-      CompView<Real> m_(m, c), d_(d, c), phi_(phi, c);
-      incrAssignUpdate(m_.v, d_.v, phi_.v);
+      CompView<Real> m_(m, c), d_(d, c);
+      CompView<double> phi_(phi, c);
+      correctUpdate(m_.v, d_.v, phi_.v, storeM);
     }
     return;
   }
-  need(d.lay, m.lay, "incrAssignUpdate");
-  need(phi.lay, m.lay, "incrAssignUpdate");
-  ops::incr_assign_update<Real>(*m.lay, m.d, d.d, phi.d);
+  need(d.lay, m.lay, "correctUpdate");
+  need(phi.lay, m.lay, "correctUpdate");
+  ops::correct_update<Real>(*m.lay, m.d, d.d, phi.d, storeM);
 }
 template <class Real>
-void AMRPoissonOp<Real>::incrPhiFromZero(T& phi, const T& x) {
+void AMRPoissonOp<Real>::incrPhiFromZero(LevelData<double>& phi, const T& x) {
   if (phi.nc > 1) {
     for (int c = 0; c < phi.nc; c++) {
-      CompView<Real> phi_(phi, c), x_(x, c);
+      CompView<double> phi_(phi, c);
+      CompView<Real> x_(x, c);
       incrPhiFromZero(phi_.v, x_.v);
     }
     return;
@@ -602,6 +604,42 @@ void AMRPoissonOp<Real>::coarseFineInterp(T& phif, const T& phic) {
   ops::cf_inhomog<Real>(m_ctx, d_cfc, n_cfc, d_cfg, d_cff, n_cff, d_deriv, phif.d, phic.d, m_dx,
                         m_refToCoarser * m_dx, m_refToCoarser);
 }
+template <class Real>
+void AMRPoissonOp<Real>::coarseFineInterpZero(T& phif) {
+  if (phif.nc > 1) {
+    for (int c = 0; c < phif.nc; c++) {
+      CompView<Real> phif_(phif, c);
+      coarseFineInterpZero(phif_.v);
+    }
+    return;
+  }
+  if (!m_coarserLay) return;
+  need(phif.lay, m_lay, "coarseFineInterp");
+  ops::cf_inhomog<Real>(m_ctx, d_cfc, n_cfc, d_cfg, d_cff, n_cff, d_deriv, phif.d, nullptr, m_dx,
+                        m_refToCoarser * m_dx, m_refToCoarser);
+}
+template <class Real>
+void AMRPoissonOp<Real>::AMRResidualZero(T& res, T& phiFine, AMRPoissonOp* finerOp) {
+  if (res.nc > 1) {
+    for (int c = 0; c < res.nc; c++) {
+      CompView<Real> res_(res, c), phiFine_(phiFine, c);
+      AMRResidualZero(res_.v, phiFine_.v, finerOp);
+    }
+    return;
+  }
+  need(res.lay, m_lay, "AMRResidual"); need(phiFine.lay, m_finerLay, "AMRResidual");
+  if (!m_vc != !finerOp->m_vc) throw std::runtime_error("reflux: variable coefficients on one level of two");
+  finerOp->coarseFineInterpZero(phiFine);
+  const double a_scale = 1.0 / m_dx;
+  if (m_vc) {
+    if (!d_vcRcFace || m_vcRefluxFine != finerOp->m_vc.get()) setupVCReflux(*finerOp->m_vc);
+    vc::reflux_zero<Real>(m_ctx, d_rcell, n_rcell, d_rf, d_vcRfFace, res.d, phiFine.d, *finerOp->m_vc,
+                          m_beta * m_refToFiner / m_dx, -a_scale);
+    return;
+  }
+  ops::reflux_residual<Real>(m_ctx, d_rcell, n_rcell, d_rc, d_rf, res.d, nullptr, phiFine.d, res.d,
+                             m_beta * 1 / m_dx, m_beta * m_refToFiner / m_dx, -a_scale, m_dx, m_alpha, m_beta);
+}
 // AMRResidual (:736-750)
 template <class Real>
 void AMRPoissonOp<Real>::AMRResidual(T& res, T& phiFine, T& phi, T& phiCoarse, const T& rhs, bool homog,
@@ -732,7 +770,8 @@ void AMRPoissonOp<Real>::AMRRestrictS(T& resCoarse, const T& residual, T& correc
                                       T& scratch) {
   if (correction.nc > 1) {
     for (int c = 0; c < correction.nc; c++) {
-      CompView<Real> resCoarse_(resCoarse, c), residual_(residual, c), correction_(correction, c), coarseCorrection_(coarseCorrection, c), scratch_(scratch, c);
+      CompView<Real> resCoarse_(resCoarse, c), residual_(residual, c), correction_(correction, c),
+          coarseCorrection_(coarseCorrection, c), scratch_(scratch, c);
       AMRRestrictS(resCoarse_.v, residual_.v, correction_.v, coarseCorrection_.v, scratch_.v);
     }
     return;
@@ -751,6 +790,12 @@ void AMRPoissonOp<Real>::AMRRestrictS(T& resCoarse, const T& residual, T& correc
   }
   AMRResidualNF(scratch, correction, coarseCorrection, residual, true);
   ops::average<Real>(*m_lay, *m_cfLay, resCoarse.d, scratch.d, m_refToCoarser);
+}
+template <class Real>
+void AMRPoissonOp<Real>::AMRRestrictSZero(T& resCoarse, const T& residual, T& correction, T& scratch) {
+  coarseFineInterpZero(correction);
+  T none;  // an undefined coarse correction: the ghosts just filled stay
+  AMRRestrictS(resCoarse, residual, correction, none, scratch);
 }
 // AMRProlongS (:959-990)
 template <class Real>
@@ -1308,14 +1353,17 @@ void AMRMultiGrid<Real>::computeAMROperator(std::vector<T*>& lphi, std::vector<T
 template <class Real>
 void AMRMultiGrid<Real>::AMRVCycle(std::vector<T*>& uberCorrection, std::vector<T*>& uberResidual, int ilev,
                                    int l_max, int l_base, bool fromZero) {
+  // fold: every level is visited once, its correction goes into phi at the end of its upsweep,
+  // and its uberCorrection, zero until then in the reference, is never read as such
+  const bool fold = !m_foldPhi.empty();
   if (ilev == l_max && l_max > l_base) {
     // (with one level the cycle works on uberCorrection / uberResidual directly and
     // the reference's copies below are never read)
     for (int level = l_base; level <= l_max; level++) {
-      if (level == l_max) {
-        // uberResidual[l_max] is read only by this copy until the next
-        // computeAMRResidual rewrites it, so the buffers trade places instead;
-        // m_correction[l_max] is first written by its relaxation from zero
+      if (level == l_max || fold) {
+        // uberResidual[level] is read only by this copy until the next computeAMRResidual
+        // rewrites it, so the buffers trade places instead; m_correction[level] is first
+        // written by its relaxation from zero
         need(m_residual[level]->lay, uberResidual[level]->lay, "AMRVCycle");
         std::swap(m_residual[level]->d, uberResidual[level]->d);
         continue;
@@ -1335,20 +1383,29 @@ void AMRMultiGrid<Real>::AMRVCycle(std::vector<T*>& uberCorrection, std::vector<
     if (fromZero) mg(l_base)->oneCycleFromZero(*m_correction[ilev], *m_residual[ilev]);
     else mg(l_base)->oneCycle(*m_correction[ilev], *m_residual[ilev]);
     // uberCorrection[l_base] is zero here and read next only by the update of phi
-    if (!m_foldPhi.empty()) m_op[ilev]->incrPhiFromZero(*m_foldPhi[ilev], *m_correction[ilev]);
+    if (fold) m_op[ilev]->incrPhiFromZero(*m_foldPhi[ilev], *m_correction[ilev]);
     else m_op[ilev]->incr(*uberCorrection[ilev], *m_correction[ilev], 1.0);
   } else {
     relax(*m_correction[ilev], *m_residual[ilev], ilev, m_pre, fromZero);
-    // on the first visit of a cycle uberCorrection[ilev] is zero (zeroed before the
-    // cycle and not written since), so the incr need not read it
-    if (fromZero) m_op[ilev]->incrFromZero(*uberCorrection[ilev], *m_correction[ilev]);
-    else m_op[ilev]->incr(*uberCorrection[ilev], *m_correction[ilev], 1.0);
-    m_op[ilev - 1]->setToZero(*m_correction[ilev - 1]);
-    std::vector<T*> res(m_residual.size());
-    for (size_t q = 0; q < res.size(); q++) res[q] = m_residual[q].get();
-    computeAMRResidualLevel(res, uberCorrection, uberResidual, l_max, l_base, ilev - 1, true);
-    m_op[ilev]->AMRRestrictS(*m_resC[ilev], *m_residual[ilev], *m_correction[ilev], *m_correction[ilev - 1],
-                             *uberCorrection[ilev]);
+    if (fold) {
+      // uberCorrection[ilev] would be the correction just relaxed, read only next to the
+      // coarse-fine interface; uberCorrection[ilev - 1] and m_correction[ilev - 1] are zero and
+      // m_residual[ilev - 1] is uberResidual[ilev - 1], so the residual of level ilev - 1
+      // differs from it in the refluxed cells only
+      m_op[ilev - 1]->AMRResidualZero(*m_residual[ilev - 1], *m_correction[ilev], m_op[ilev].get());
+      m_op[ilev]->AMRRestrictSZero(*m_resC[ilev], *m_residual[ilev], *m_correction[ilev], *uberCorrection[ilev]);
+    } else {
+      // on the first visit of a cycle uberCorrection[ilev] is zero (zeroed before the
+      // cycle and not written since), so the incr need not read it
+      if (fromZero) m_op[ilev]->incrFromZero(*uberCorrection[ilev], *m_correction[ilev]);
+      else m_op[ilev]->incr(*uberCorrection[ilev], *m_correction[ilev], 1.0);
+      m_op[ilev - 1]->setToZero(*m_correction[ilev - 1]);
+      std::vector<T*> res(m_residual.size());
+      for (size_t q = 0; q < res.size(); q++) res[q] = m_residual[q].get();
+      computeAMRResidualLevel(res, uberCorrection, uberResidual, l_max, l_base, ilev - 1, true);
+      m_op[ilev]->AMRRestrictS(*m_resC[ilev], *m_residual[ilev], *m_correction[ilev], *m_correction[ilev - 1],
+                               *uberCorrection[ilev]);
+    }
     m_op[ilev - 1]->assignCopier(*m_residual[ilev - 1], *m_resC[ilev]);
     for (int img = 0; img < m_numMG; img++)
       AMRVCycle(uberCorrection, uberResidual, ilev - 1, l_max, l_base, img == 0);
@@ -1358,11 +1415,23 @@ void AMRMultiGrid<Real>::AMRVCycle(std::vector<T*>& uberCorrection, std::vector<
     relax(dCorr, *m_residual[ilev], ilev, m_post, true);  // setToZero(dCorr) + relax
     // incr(m_correction, dCorr, 1.0) then assignLocal(uberCorrection, m_correction),
     // in one pass over the valid cells (every later read of a ghost refills it);
-    // with the phi update folded in, uberCorrection[ilev] is read next only by
-    // solveNoInitResid's incr(phi) and setToZero, which this pass performs too
-    if (!m_foldPhi.empty()) m_op[ilev]->incrAssignUpdate(*m_correction[ilev], dCorr, *m_foldPhi[ilev]);
+    // with the phi update folded in, the sum goes into phi at once, and into m_correction only
+    // where a finer level reads it
+    if (fold) m_op[ilev]->correctUpdate(*m_correction[ilev], dCorr, *m_foldPhi[ilev], ilev < l_max);
     else m_op[ilev]->incrAssign(*m_correction[ilev], dCorr);
   }
+}
+template <class Real>
+void AMRMultiGrid<Real>::foldedVCycle(std::vector<LevelData<double>*>& phi, std::vector<T*>& uberCorrection,
+                                      std::vector<T*>& uberResidual, int l_max, int l_base) {
+  m_foldPhi.assign(phi.begin(), phi.end());
+  try {
+    AMRVCycle(uberCorrection, uberResidual, l_max, l_max, l_base);
+  } catch (...) {
+    m_foldPhi.clear();
+    throw;
+  }
+  m_foldPhi.clear();
 }
 // solveNoInitResid (AMRMultiGrid.H:935-1124)
 template <class Real>
@@ -1374,10 +1443,11 @@ void AMRMultiGrid<Real>::solveNoInitResid(std::vector<T*>& phi, std::vector<T*>&
   // with l_base > 0 the residual of level l_base takes coarse-fine data from the
   // uberCorrection one level lower, which stays zero (AMRMultiGrid.H:952-967)
   if (l_base > 0) m_op[l_base - 1]->setToZero(*uberCorrection[l_base - 1]);
-  for (int ilev = l_base; ilev <= l_max; ilev++) {
-    m_op[ilev]->setToZero(*uberResidual[ilev]);
-    m_op[ilev]->setToZero(*uberCorrection[ilev]);
-  }
+  // (uberResidual is written whole before it is read; uberCorrection is read as zero only where
+  // the update of phi is not folded into the cycle)
+  const bool folds = m_innerCycleUpdate || (m_numMG == 1 && l_max > l_base);
+  if (!folds)
+    for (int ilev = l_base; ilev <= l_max; ilev++) m_op[ilev]->setToZero(*uberCorrection[ilev]);
   if (zeroPhi)
     for (int ilev = l_base; ilev <= l_max; ilev++) m_op[ilev]->setToZero(*phi[ilev]);
   m_initial_rnorm = computeAMRResidual(uberResidual, phi, rhs, l_max, l_base, false, true);
@@ -1395,14 +1465,8 @@ void AMRMultiGrid<Real>::solveNoInitResid(std::vector<T*>& phi, std::vector<T*>&
     } else if (m_numMG == 1 && l_max > l_base) {
       // every level is visited once per cycle: its correction goes into phi at the
       // end of its upsweep, with the arithmetic of the update below
-      m_foldPhi.assign(phi.begin(), phi.end());
-      try {
-        AMRVCycle(uberCorrection, uberResidual, l_max, l_max, l_base);
-      } catch (...) {
-        m_foldPhi.clear();
-        throw;
-      }
-      m_foldPhi.clear();
+      if constexpr (sizeof(Real) == 8) foldedVCycle(phi, uberCorrection, uberResidual, l_max, l_base);
+      else throw std::runtime_error("solveNoInitResid: the outer iteration is FP64");
     } else {
       AMRVCycle(uberCorrection, uberResidual, l_max, l_max, l_base);
       for (int ilev = l_base; ilev <= l_max; ilev++) {

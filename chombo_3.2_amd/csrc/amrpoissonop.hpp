@@ -93,8 +93,12 @@ class AMRPoissonOp : public AMRLevelOp<LevelData<Real>> {
   // lhs = lhs + x * 1.0 then x = lhs on the valid cells (incr + assignLocal fused)
   void incrAssign(T& lhs, T& x);
   void incrFromZero(T& lhs, const T& x);
-  void incrAssignUpdate(T& m, T& d, T& phi);
-  void incrPhiFromZero(T& phi, const T& x);
+  // v = m + d, phi += v (and m = v with storeM); phi += x: the V-cycle's updates of the FP64 phi
+  void correctUpdate(T& m, const T& d, LevelData<double>& phi, bool storeM);
+  void incrPhiFromZero(LevelData<double>& phi, const T& x);
+  // AMRResidual / AMRResidualNC of a zero phi (and a zero phiCoarse) where res holds rhs: only
+  // the refluxed cells change
+  void AMRResidualZero(T& res, T& phiFine, AMRPoissonOp* finerOp);
   void axby(T& lhs, const T& x, const T& y, double a, double b) override;
   void scale(T& lhs, double s) override;
   double norm(const T& x, int ord) override;
@@ -129,6 +133,9 @@ class AMRPoissonOp : public AMRLevelOp<LevelData<Real>> {
   void levelGSRB(T& phi, const T& rhs);
   void homogeneousCFInterp(T& phi);
   void coarseFineInterp(T& phif, const T& phic);   // QuadCFInterp of this level from the coarser one
+  void coarseFineInterpZero(T& phif);              // the same from a zero coarser field
+  // AMRRestrictS with a coarse correction that is zero (it is not read)
+  void AMRRestrictSZero(T& resCoarse, const T& residual, T& correction, T& scratch);
   void reflux(T& phiFine, T& phi, T& res, AMRPoissonOp* finerOp);
   void residualFused(T& res, T& phiFine, T& phi, const T& rhs, bool homog, AMRPoissonOp* finerOp);
   void localMaxNormAsync(const T& x, int slot, bool accumulate);
@@ -235,10 +242,10 @@ class AMRMultiGrid {
   // m_innerBottomMetrics receives the bottom solver's convergence metrics.
   std::function<void(std::vector<T*>&, std::vector<T*>&, int, int)> m_innerCycleUpdate;
   std::function<void(double, double)> m_innerBottomMetrics;
-  // While solveNoInitResid runs a V-cycle with the phi update folded in (one
-  // coarser cycle per level, FP64 update): the phi of every level.  The cycle then
-  // adds each level's correction to phi itself and leaves uberCorrection zero.
-  std::vector<T*> m_foldPhi;
+  // While a V-cycle runs that visits every level once (m_numMG 1, l_max > l_base): the FP64 phi
+  // of every level.  The cycle then adds each level's correction to phi itself, uses
+  // uberCorrection as scratch only and trades its residual buffers with uberResidual's.
+  std::vector<LevelData<double>*> m_foldPhi;
 
   void define(AMRPoissonOpFactory<Real>& factory, LinearSolver<T>* bottom, int numLevels);
   void setSolverParameters(int pre, int post, int bottom, int numMG, int iterMax, double eps, double hang,
@@ -248,6 +255,9 @@ class AMRMultiGrid {
                         std::vector<T*>& rhs, int l_max, int l_base, bool zeroPhi);
   void AMRVCycle(std::vector<T*>& uberCorrection, std::vector<T*>& uberResidual, int ilev, int l_max, int l_base,
                  bool fromZero = true);
+  // one V-cycle with m_foldPhi = phi (m_numMG must be 1 and l_max > l_base)
+  void foldedVCycle(std::vector<LevelData<double>*>& phi, std::vector<T*>& uberCorrection,
+                    std::vector<T*>& uberResidual, int l_max, int l_base);
   double computeAMRResidual(std::vector<T*>& resid, std::vector<T*>& phi, std::vector<T*>& rhs, int l_max,
                             int l_base, bool homogeneousBC, bool computeNorm);
   void computeAMRResidualLevel(std::vector<T*>& resid, std::vector<T*>& phi, std::vector<T*>& rhs, int l_max,

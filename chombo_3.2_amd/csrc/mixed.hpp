@@ -104,10 +104,12 @@ struct MixedInner {
   void cycle(std::vector<LevelData<double>*>& phi, std::vector<LevelData<double>*>& ur, int l_max, int l_base) {
     std::vector<LevelData<float>*> c, r;
     for (size_t l = 0; l < corr.size(); l++) { c.push_back(corr[l].get()); r.push_back(res[l].get()); }
-    for (int l = l_base; l <= l_max; l++) {
-      ops::convert_valid_d2f(*ur[l]->lay, r[l]->d, ur[l]->d);
-      ops::setval<float>(*c[l]->lay, c[l]->d, 0.0);
+    for (int l = l_base; l <= l_max; l++) ops::convert_valid_d2f(*ur[l]->lay, r[l]->d, ur[l]->d);
+    if (amg.m_numMG == 1 && l_max > l_base) {
+      amg.foldedVCycle(phi, c, r, l_max, l_base);
+      return;
     }
+    for (int l = l_base; l <= l_max; l++) ops::setval<float>(*c[l]->lay, c[l]->d, 0.0);
     amg.AMRVCycle(c, r, l_max, l_max, l_base);
     for (int l = l_base; l <= l_max; l++) ops::update_f2d(*phi[l]->lay, phi[l]->d, c[l]->d);
   }

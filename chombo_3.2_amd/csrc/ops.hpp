@@ -119,12 +119,13 @@ void incr_assign(const DeviceLayout& L, T* lhs, T* x);
 // lhs = 0 + x * 1 (setToZero then incr, lhs not read)
 template <class T>
 void incr_from_zero(const DeviceLayout& L, T* lhs, const T* x);
-// m += d; d = m; phi += d; d = 0 (incr, assignLocal, incr, setToZero)
+// v = m + d; phi += v, and m = v with store_m (incr, assignLocal, incr of a correction that is
+// read later through m, if at all); phi is FP64 also for FP32 corrections (phi += (0 + v) * 1)
 template <class T>
-void incr_assign_update(const DeviceLayout& L, T* m, T* d, T* phi);
+void correct_update(const DeviceLayout& L, T* m, const T* d, double* phi, bool store_m);
 // phi += (0 + x * 1) * 1 (an incr into a zero field, then into phi)
 template <class T>
-void incr_phi_from_zero(const DeviceLayout& L, T* phi, const T* x);
+void incr_phi_from_zero(const DeviceLayout& L, double* phi, const T* x);
 template <class T>
 void axby(const DeviceLayout& L, T* lhs, const T* x, const T* y, double a, double b);
 template <class T>
@@ -168,14 +169,16 @@ double norm1_ordered(const DeviceLayout& L, const T* x, int slot, int nc = 1, lo
 template <class T>
 void maxnorm_async(const DeviceLayout& L, const T* x, int slot, int accumulate);
 
-// inhomogeneous coarse-fine interpolation (QuadCFInterp::coarseFineInterp)
+// inhomogeneous coarse-fine interpolation (QuadCFInterp::coarseFineInterp); phic null: the
+// coarser field is zero (its derivatives are not formed)
 template <class T>
 void cf_inhomog(Context* ctx, const CFCoarse* dc, int ncoarse, const CFGen* dg, const CFFine* df, int nfine,
                 T* deriv_scratch, T* phif, const T* phic, double dxf, double dxc, int nref = 2);
 
 // AMRResidual's AMROperator + axby(res, res, rhs, -1, 1) in two launches: every valid
 // cell from its stencil, then the refluxed cells again with their corrections;
-// bitwise the operator, reflux and axby launches
+// bitwise the operator, reflux and axby launches.  reflux_residual with phic null: the level's
+// own field is zero (res elsewhere is then rhs as it is)
 template <class T>
 void apply_residual(const DeviceLayout& L, T* res, const T* phi, const T* rhs, double dx, double alpha, double beta);
 template <class T>

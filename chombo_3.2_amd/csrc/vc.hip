@@ -756,8 +756,8 @@ __global__ void __launch_bounds__(256) k_vc_reflux(const RefluxCell* __restrict_
   const int r = blockIdx.x * 256 + threadIdx.x;
   if (r >= n) return;
   const RefluxCell c = cells[r];
-  T val = u[c.u];
-  if (c.nc > 0) {
+  T val = phic ? u[c.u] : T(0.0);  // phic null: the level's field is zero (see reflux_zero)
+  if (phic && c.nc > 0) {
     T reg = T(0.0);
     for (int q = c.c0; q < c.c0 + c.nc; q++) {
       const RefluxCoarse x = rc[q];
@@ -780,7 +780,7 @@ __global__ void __launch_bounds__(256) k_vc_reflux(const RefluxCell* __restrict_
     }
     if (x.last) val = val + freg * minus_s;
   }
-  u[c.u] = val;
+  u[c.u] = phic ? val : val * T(-1.0) + u[c.u] * T(1.0);
 }
 template <class T>
 void reflux(Context* ctx, const RefluxCell* cells, int ncells, const RefluxCoarse* rc, const RefluxFine* rf,
@@ -791,6 +791,19 @@ void reflux(Context* ctx, const RefluxCell* cells, int ncells, const RefluxCoars
   hipEvent_t ev = profile_begin(ctx, KC_REFLUX);
   hipLaunchKernelGGL(k_vc_reflux<T>, dim3((ncells + 255) / 256), dim3(256), 0, ctx->stream, cells, ncells, rc, rf, fc,
                      ff, u, phic, phif, bc, bf, T(beta_dx_c), T(beta_ref_dx_c), T(minus_inv_dx));
+  hip_check(hipGetLastError(), "k_vc_reflux");
+  profile_end(ctx, ev, KC_REFLUX, 0.0);
+}
+
+template <class T>
+void reflux_zero(Context* ctx, const RefluxCell* cells, int ncells, const RefluxFine* rf, const VCFaceIdx* ff, T* u,
+                 const T* phif, const VCCoefs<T>& F, double beta_ref_dx_c, double minus_inv_dx) {
+  if (ncells <= 0 || ctx->dry) return;
+  VCB3<T> bf{{F.b[0], F.b[1], F.b[2]}};
+  hipEvent_t ev = profile_begin(ctx, KC_REFLUX);
+  hipLaunchKernelGGL(k_vc_reflux<T>, dim3((ncells + 255) / 256), dim3(256), 0, ctx->stream, cells, ncells,
+                     (const RefluxCoarse*)nullptr, rf, (const VCFaceIdx*)nullptr, ff, u, (const T*)nullptr, phif,
+                     VCB3<T>{}, bf, T(0.0), T(beta_ref_dx_c), T(minus_inv_dx));
   hip_check(hipGetLastError(), "k_vc_reflux");
   profile_end(ctx, ev, KC_REFLUX, 0.0);
 }
@@ -822,7 +835,9 @@ void narrow(const VCCoefs<double>& src, VCCoefs<float>& dst) {
   template void scale_by_lambda<T>(const DeviceLayout&, const VCCoefs<T>&, T*);                                     \
   template void reflux<T>(Context*, const RefluxCell*, int, const RefluxCoarse*, const RefluxFine*, const VCFaceIdx*, \
                           const VCFaceIdx*, T*, const T*, const T*, const VCCoefs<T>&, const VCCoefs<T>&, double,     \
-                          double, double);
+                          double, double);                                                                       \
+  template void reflux_zero<T>(Context*, const RefluxCell*, int, const RefluxFine*, const VCFaceIdx*, T*, const T*, \
+                               const VCCoefs<T>&, double, double);
 VC_INST(double)
 VC_INST(float)
 

@@ -87,6 +87,11 @@ template <class T>
 void reflux(Context* ctx, const RefluxCell* cells, int ncells, const RefluxCoarse* rc, const RefluxFine* rf,
             const VCFaceIdx* fc, const VCFaceIdx* ff, T* u, const T* phic, const T* phif, const VCCoefs<T>& C,
             const VCCoefs<T>& F, double beta_dx_c, double beta_ref_dx_c, double minus_inv_dx);
+// the refluxed cells of the residual of a zero field: u = u - (reflux corrections), which is
+// reflux of the zero operator values followed by axby(u, ., rhs, -1, 1) where u holds rhs
+template <class T>
+void reflux_zero(Context* ctx, const RefluxCell* cells, int ncells, const RefluxFine* rf, const VCFaceIdx* ff, T* u,
+                 const T* phif, const VCCoefs<T>& F, double beta_ref_dx_c, double minus_inv_dx);
 // diagonalScale / divideByIdentityCoef (VCAMRPoissonOp2.H:120-140): x *= aCoef,
 // resp. x /= aCoef on valid cells
 template <class T>
