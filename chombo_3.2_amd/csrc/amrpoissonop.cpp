@@ -3,6 +3,8 @@
 // AMRMultiGrid.H; each method cites the reference lines it follows.
 #include "amrpoissonop.hpp"
 
+#include "block.hpp"
+
 #include <cmath>
 #include <stdexcept>
 
@@ -417,13 +419,56 @@ bool AMRPoissonOp<Real>::tuneRelax(const T& phi, const T& rhs, double* times) {
       ops::tune_gsrb_fused<Real>(*m_lay, m_faces, m_relaxTmp.d, phi.d, rhs.d, m_dx, m_alpha, m_beta, times);
   m_relaxShape = pick.first;
   m_relaxKc = pick.second;
+  m_shapeSet = false;
   return true;
+}
+template <class Real>
+bool AMRPoissonOp<Real>::blockVisits() const {
+  return m_fused && m_ctx->fused_relax && !m_vc && m_relaxMode == 1 && !m_shapeSet && ops::block_visit_ok(*m_lay);
+}
+template <class Real>
+void AMRPoissonOp<Real>::relaxBlocks(T& e, const T& r, int n, bool fromZero, const T* coarse, T* resc) {
+  need(e.lay, m_lay, "relax"); need(r.lay, m_lay, "relax");
+  if (coarse) need(coarse->lay, m_mgCoarse, "prolongIncrement");
+  if (resc) need(resc->lay, m_mgCoarse, "restrictResidual");
+  if (r.nc != e.nc || (coarse && coarse->nc != e.nc) || (resc && resc->nc != e.nc))
+    throw std::runtime_error("levelGSRB: component counts differ");
+  if (!e.own) throw std::runtime_error("levelGSRB: the one-launch relaxation swaps buffers and takes whole fields");
+  T& tmp = e.nc > 1 ? m_relaxTmpN : m_relaxTmp;
+  if (!tmp.isDefined() || tmp.nc != e.nc) tmp.define(m_lay, e.nc);
+  if (e.nc > 1 && (tmp.cs != e.cs || r.cs != e.cs)) throw std::runtime_error("levelGSRB: component strides differ");
+  for (int done = 0; done < n;) {
+    // an odd count starts with one iteration, so that the last visit has two
+    const int sweeps = (n - done) % 2 ? 1 : 2;
+    const bool first = done == 0, last = done + sweeps == n;
+    for (int c = 0; c < e.nc; c++)
+      ops::block_visit<Real>(*m_lay, m_faces, m_mgCoarse, tmp.d + c * e.cs, e.d + c * e.cs, r.d + c * e.cs,
+                             first && coarse ? coarse->d + c * coarse->cs : nullptr,
+                             last && resc ? resc->d + c * resc->cs : nullptr, m_dx, m_alpha, m_beta, sweeps,
+                             first && fromZero);
+    std::swap(e.d, tmp.d);
+    done += sweeps;
+  }
+}
+template <class Real>
+void AMRPoissonOp<Real>::relaxRestrict(T& e, const T& r, int n, bool fromZero, T& resc) {
+  if (n > 0 && blockVisits()) relaxBlocks(e, r, n, fromZero, nullptr, &resc);
+  else MGLevelOp<T>::relaxRestrict(e, r, n, fromZero, resc);
+}
+template <class Real>
+void AMRPoissonOp<Real>::prolongRelax(T& e, const T& c, const T& r, int n) {
+  if (n > 0 && blockVisits()) relaxBlocks(e, r, n, false, &c, nullptr);
+  else MGLevelOp<T>::prolongRelax(e, c, r, n);
 }
 // setToZero + relax: on merged levels the first iteration reads no old values
 // (they are all zero) and writes every valid cell, so the zeroing itself is
 // dropped; ghost cells are refilled before any later read, as after any relax.
 template <class Real>
 void AMRPoissonOp<Real>::relaxFromZero(T& e, const T& r, int n) {
+  if (n > 0 && blockVisits()) {
+    relaxBlocks(e, r, n, true, nullptr, nullptr);
+    return;
+  }
   if (!(m_fused && m_ctx->fused_relax) || m_vc || m_relaxMode != 1 || n <= 0 || e.nc > 1) {
     setToZero(e);
     relax(e, r, n);
@@ -443,6 +488,10 @@ void AMRPoissonOp<Real>::relax(T& e, const T& r, int n) {
       CompView<Real> e_(e, c), r_(r, c);
       relax(e_.v, r_.v, n);
     }
+    return;
+  }
+  if (n > 0 && e.own && blockVisits()) {
+    relaxBlocks(e, r, n, false, nullptr, nullptr);
     return;
   }
   for (int i = 0; i < n; i++) {

@@ -32,7 +32,14 @@ class AMRPoissonOp : public AMRLevelOp<LevelData<Real>> {
   // second buffer it relaxes into, swapped with the relaxed field afterwards
   bool m_fused = false;
   ops::FaceRules m_faces{};
-  int m_relaxShape = 0, m_relaxKc = 0;        // tile shape and z-chunk (0: automatic), see tuneRelax
+  int m_relaxShape = -1, m_relaxKc = 0;       // tile shape (-1: by size) and z-chunk (0: automatic), see tuneRelax
+  bool m_shapeSet = false;                    // the tile shape was asked for, not timed or chosen by size
+  // whether this level's smoothing visits run as blocks (block.hpp): small, one-launch
+  // relaxation, levelGSRB, no tile shape asked for
+  bool blockVisits() const;
+  // n > 0 GSRB iterations of e in block visits: from zero, after the prolongation of coarse, with
+  // the restriction of the result to resc (each where given)
+  void relaxBlocks(T& e, const T& r, int n, bool fromZero, const T* coarse, T* resc);
   LevelData<Real> m_relaxTmp;
   LevelData<Real> m_relaxTmpN;                // the same for fields of several components
   // coarser AMR level (QuadCFInterp + restriction/prolongation copiers)
@@ -108,6 +115,8 @@ class AMRPoissonOp : public AMRLevelOp<LevelData<Real>> {
   void createCoarser(T& coarse, const T& fine, bool ghosted) override;
   void relax(T& correction, const T& residual, int iterations) override;
   void relaxFromZero(T& correction, const T& residual, int iterations) override;
+  void relaxRestrict(T& correction, const T& residual, int iterations, bool fromZero, T& resCoarse) override;
+  void prolongRelax(T& correction, const T& correctCoarse, const T& residual, int iterations) override;
   void restrictResidual(T& resCoarse, T& phiFine, const T& rhsFine) override;
   void prolongIncrement(T& phiThisLevel, const T& correctCoarse) override;
   // ---- AMRLevelOp ----

@@ -694,6 +694,7 @@ int amrmg_solver_set_relax_shape(amrmg_solver* s, int shape, int kc) {
     if (!ops::fused_shape_ok(shape, bytes, op->m_lay->rect.len(0))) return;
     op->m_relaxShape = shape;
     op->m_relaxKc = kc;
+    op->m_shapeSet = true;
   };
   for (int l = 0; l < s->nlev(); l++) set(s->amg.m_op[l].get(), 8);
   for (int d = 1; d < s->H.mgDepth(); d++) set(s->mgop(d), 8);

@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <utility>
 
 namespace amrmg {
 namespace ops {
@@ -276,6 +277,17 @@ constexpr int kFusedShapeTable[][4] = {
 // (scheme 2: FP32, nx a multiple of 4).
 inline bool fused_shape_ok(int shape, int elem_bytes, int nx) {
   return kFusedShapeTable[shape][3] != 2 || (elem_bytes == 4 && nx % 4 == 0);
+}
+// The tile shape and z-chunk used where none is asked for, by the level's cells (with
+// measured microseconds per FP64 iteration against the former default, 64 x 8 columns of five LDS
+// planes): up to 1 million cells 32 x 10 x-pair columns in short chunks (64^3: 6.6, was 12.3;
+// 96^3: 8.9, was 16.7), up to 12 million 32 x 24 in chunks of 8 planes (128^3: 13.7, was 20.0; 216 x
+// 160 x 200: 31.5, was 62.2), above that 64 x 11 in chunks of 32 (256^3: 100, was 114; 320^3: 180,
+// was 202).  FP32 takes the same shapes (128^3: 10.5, was 17.2; 256^3: 36.4, was 64.8).
+inline std::pair<int, int> default_relax_shape(long long cells) {
+  if (cells <= (1LL << 20)) return {16, 0};
+  if (cells <= 12LL << 20) return {14, 8};
+  return {15, 32};
 }
 // x-quad rows: quads start at lo[0] - 2 (one value precedes the first row) and the
 // one holding hi[0] ends at hi[0] + 2 (rows padded by at least 4 values)

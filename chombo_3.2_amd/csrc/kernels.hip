@@ -743,9 +743,14 @@ static void launch_fused(Context* ctx, int shape, int grid, const FusedArgs& a, 
   prof_end(ctx, ev, KC_GSRB, bytes, units);
 }
 
-static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int shape, int kc, bool zero_src,
+static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int& shape, int kc, bool zero_src,
                             int elem_bytes) {
   if (!L.merged) throw std::runtime_error("gsrb_fused: level is not stored merged");
+  if (shape < 0) {
+    const std::pair<int, int> s = default_relax_shape(L.valid_cells);
+    shape = s.first;
+    if (kc <= 0) kc = s.second;
+  }
   if (shape < 0 || shape >= kNumFusedShapes) throw std::runtime_error("gsrb_fused: bad tile shape");
   if (!fused_shape_ok(shape, elem_bytes, L.rect.len(0)))
     throw std::runtime_error("gsrb_fused: x-quad tile shapes need FP32 and an x extent that is a multiple of 4");

@@ -49,6 +49,18 @@ class MGLevelOp : public LinearOp<T> {
   }
   virtual void restrictResidual(T& resCoarse, T& phiFine, const T& rhsFine) = 0;
   virtual void prolongIncrement(T& phiThisLevel, const T& correctCoarse) = 0;
+  // A V-cycle's visit of this level on the way down, (setToZero with fromZero and) relax then
+  // restrictResidual, and on the way up, prolongIncrement then relax; an operator may do each
+  // in fewer steps with the same values
+  virtual void relaxRestrict(T& correction, const T& residual, int iterations, bool fromZero, T& resCoarse) {
+    if (fromZero) relaxFromZero(correction, residual, iterations);
+    else relax(correction, residual, iterations);
+    restrictResidual(resCoarse, correction, residual);
+  }
+  virtual void prolongRelax(T& correction, const T& correctCoarse, const T& residual, int iterations) {
+    prolongIncrement(correction, correctCoarse);
+    relax(correction, residual, iterations);
+  }
 };
 
 template <class T>
@@ -291,14 +303,12 @@ class MultiGrid {
       m_op[depth]->relax(correction, residual, m_post);
       return;
     }
-    relax(m_pre);
-    m_op[depth]->restrictResidual(*m_residual[depth + 1], correction, residual);
+    m_op[depth]->relaxRestrict(correction, residual, m_pre, zero, *m_residual[depth + 1]);
     // setToZero(m_correction[depth + 1]) is folded into the first coarser cycle's
     // first relaxation (relaxFromZero)
     for (int img = 0; img < cycles; img++)
       cycle(depth + 1, *m_correction[depth + 1], *m_residual[depth + 1], img == 0);
-    m_op[depth]->prolongIncrement(correction, *m_correction[depth + 1]);
-    m_op[depth]->relax(correction, residual, m_post);
+    m_op[depth]->prolongRelax(correction, *m_correction[depth + 1], residual, m_post);
   }
 };
 
