@@ -423,6 +423,24 @@ bool AMRPoissonOp<Real>::tuneRelax(const T& phi, const T& rhs, double* times) {
   return true;
 }
 template <class Real>
+bool AMRPoissonOp<Real>::pairMarches() const {
+  return m_fused && m_ctx->fused_relax && !m_vc && m_relaxMode == 1 && !m_shapeSet && !ops::block_visit_ok(*m_lay);
+}
+template <class Real>
+void AMRPoissonOp<Real>::relaxPairs(T& e, const T& r, int pairs, bool zero) {
+  need(e.lay, m_lay, "relax"); need(r.lay, m_lay, "relax");
+  if (r.nc != e.nc) throw std::runtime_error("levelGSRB: component counts differ");
+  T& tmp = e.nc > 1 ? m_relaxTmpN : m_relaxTmp;
+  if (!tmp.isDefined() || tmp.nc != e.nc) tmp.define(m_lay, e.nc);
+  if (e.nc > 1 && (tmp.cs != e.cs || r.cs != e.cs)) throw std::runtime_error("levelGSRB: component strides differ");
+  for (int q = 0; q < pairs; q++) {
+    for (int c = 0; c < e.nc; c++)
+      ops::gsrb_two<Real>(*m_lay, m_faces, tmp.d + c * e.cs, e.d + c * e.cs, r.d + c * e.cs, m_dx, m_alpha, m_beta,
+                          zero && q == 0);
+    std::swap(e.d, tmp.d);
+  }
+}
+template <class Real>
 bool AMRPoissonOp<Real>::blockVisits() const {
   return m_fused && m_ctx->fused_relax && !m_vc && m_relaxMode == 1 && !m_shapeSet && ops::block_visit_ok(*m_lay);
 }
@@ -469,6 +487,11 @@ void AMRPoissonOp<Real>::relaxFromZero(T& e, const T& r, int n) {
     relaxBlocks(e, r, n, true, nullptr, nullptr);
     return;
   }
+  if (n > 1 && e.own && pairMarches()) {
+    relaxPairs(e, r, n / 2, true);
+    if (n % 2) relax(e, r, 1);
+    return;
+  }
   if (!(m_fused && m_ctx->fused_relax) || m_vc || m_relaxMode != 1 || n <= 0 || e.nc > 1) {
     setToZero(e);
     relax(e, r, n);
@@ -493,6 +516,10 @@ void AMRPoissonOp<Real>::relax(T& e, const T& r, int n) {
   if (n > 0 && e.own && blockVisits()) {
     relaxBlocks(e, r, n, false, nullptr, nullptr);
     return;
+  }
+  if (n > 1 && e.own && pairMarches()) {
+    relaxPairs(e, r, n / 2, false);
+    n %= 2;
   }
   for (int i = 0; i < n; i++) {
     if (m_relaxMode == 4) levelJacobi(e, r);

@@ -37,6 +37,10 @@ class AMRPoissonOp : public AMRLevelOp<LevelData<Real>> {
   // whether this level's smoothing visits run as blocks (block.hpp): small, one-launch
   // relaxation, levelGSRB, no tile shape asked for
   bool blockVisits() const;
+  // whether pairs of GSRB iterations run as one march: the larger levels on the same terms
+  bool pairMarches() const;
+  // from zero (zero) or from e, `pairs` pairs of GSRB iterations
+  void relaxPairs(T& e, const T& r, int pairs, bool zero);
   // n > 0 GSRB iterations of e in block visits: from zero, after the prolongation of coarse, with
   // the restriction of the result to resc (each where given)
   void relaxBlocks(T& e, const T& r, int n, bool fromZero, const T* coarse, T* resc);

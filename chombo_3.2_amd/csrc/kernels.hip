@@ -19,7 +19,7 @@
 
 #include "fused.hpp"
 #include "ops.hpp"
-#include "zmarch.hpp"
+#include "zmarch2.hpp"
 
 namespace amrmg {
 
@@ -743,18 +743,10 @@ static void launch_fused(Context* ctx, int shape, int grid, const FusedArgs& a, 
   prof_end(ctx, ev, KC_GSRB, bytes, units);
 }
 
-static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int& shape, int kc, bool zero_src,
-                            int elem_bytes) {
+// the work of a level's rectangle in columns of FX x FY cells and z-chunks of kc planes (0: as
+// long as amortises the 2-plane prologue while the chunks fill the chip)
+static FusedArgs tile_args(const DeviceLayout& L, const FaceRules& fr, int FX, int FY, int kc, bool zero_src) {
   if (!L.merged) throw std::runtime_error("gsrb_fused: level is not stored merged");
-  if (shape < 0) {
-    const std::pair<int, int> s = default_relax_shape(L.valid_cells);
-    shape = s.first;
-    if (kc <= 0) kc = s.second;
-  }
-  if (shape < 0 || shape >= kNumFusedShapes) throw std::runtime_error("gsrb_fused: bad tile shape");
-  if (!fused_shape_ok(shape, elem_bytes, L.rect.len(0)))
-    throw std::runtime_error("gsrb_fused: x-quad tile shapes need FP32 and an x extent that is a multiple of 4");
-  const int FX = kFusedShapeTable[shape][0], FY = kFusedShapeTable[shape][1];
   const DBox& R = L.h_boxes[L.nbox];
   FusedArgs a;
   for (int q = 0; q < 3; q++) { a.lo[q] = R.lo[q]; a.hi[q] = R.hi[q]; }
@@ -767,13 +759,11 @@ static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int& sha
   a.sy = R.sy;
   a.sz = R.sz;
   check_pair_rows(a);
-  if (kFusedShapeTable[shape][3] == 2) check_quad_rows(a);
   a.zsrc = zero_src ? 1 : 0;
   a.ntx = (L.rect.len(0) + FX - 1) / FX;
   a.nty = (L.rect.len(1) + FY - 1) / FY;
   const int nz = L.rect.len(2);
   if (kc <= 0) {
-    // z-chunks: long enough to amortise the 2-plane prologue, enough of them to fill the chip
     kc = 32;
     while (kc > 4 && (long long)a.ntx * a.nty * ((nz + kc - 1) / kc) < 2048) kc >>= 1;
   }
@@ -781,6 +771,20 @@ static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int& sha
   const long long nwork = (long long)a.ntx * a.nty * ((nz + kc - 1) / kc);
   if (nwork > INT32_MAX - 8) throw std::runtime_error("gsrb_fused: level too large");
   a.nwork = (int)nwork;
+  return a;
+}
+static FusedArgs fused_args(const DeviceLayout& L, const FaceRules& fr, int& shape, int kc, bool zero_src,
+                            int elem_bytes) {
+  if (shape < 0) {
+    const std::pair<int, int> s = default_relax_shape(L.valid_cells);
+    shape = s.first;
+    if (kc <= 0) kc = s.second;
+  }
+  if (shape < 0 || shape >= kNumFusedShapes) throw std::runtime_error("gsrb_fused: bad tile shape");
+  if (!fused_shape_ok(shape, elem_bytes, L.rect.len(0)))
+    throw std::runtime_error("gsrb_fused: x-quad tile shapes need FP32 and an x extent that is a multiple of 4");
+  const FusedArgs a = tile_args(L, fr, kFusedShapeTable[shape][0], kFusedShapeTable[shape][1], kc, zero_src);
+  if (kFusedShapeTable[shape][3] == 2) check_quad_rows(a);
   return a;
 }
 
@@ -808,6 +812,66 @@ void gsrb_fused(const DeviceLayout& L, const FaceRules& fr, T* dst, const T* src
     launch_fused<T, false>(L.ctx, shape, grid, a, dst, src, rhs, T(dxinv), T(lambda), T(alpha), T(beta), c1, c2,
                            bytes, units);
 }
+
+// two iterations in one march (zmarch2.hpp)
+template <class T, bool LAP, int FX, int FY, int NT, bool ZSRC>
+__global__ void __launch_bounds__(NT) k_gsrb_zmarch2(FusedArgs a, T* __restrict__ dst, const T* __restrict__ src,
+                                                      const T* __restrict__ rhs, T dxinv, T lambda, T alpha, T beta,
+                                                      T c1, T c2) {
+  const int w = xcd_contiguous_block();
+  if (w >= a.nwork) return;
+  zmarch2_body<T, LAP, FX, FY, NT, 2, ZSRC>(a, w, dst, src, rhs, dxinv, lambda, alpha, beta, c1, c2);
+}
+template <class T, int FX, int FY, int NT>
+static void launch_two(const DeviceLayout& L, const FaceRules& fr, T* dst, const T* src, const T* rhs, double dx,
+                       double alpha, double beta, int kc, bool zero_src) {
+  const FusedArgs a = tile_args(L, fr, FX, FY, kc, zero_src);
+  const int grid = (a.nwork + 7) / 8 * 8;
+  const double dxinv = 1.0 / (dx * dx);
+  double sum_b = 0.0;
+  for (int d = 0; d < 3; d++) sum_b = sum_b + 2.0 * dxinv;
+  const bool lap = (alpha == 0.0 && beta == 1.0);
+  const double lambda = lap ? -1.0 / sum_b : -1.0 / (alpha - beta * sum_b);
+  hipEvent_t ev = prof_begin(L.ctx, KC_GSRB);
+#define TWO_LAUNCH(LAP, Z)                                                                                       \
+  hipLaunchKernelGGL((k_gsrb_zmarch2<T, LAP, FX, FY, NT, Z>), dim3(grid), dim3(NT), 0, L.ctx->stream, a, dst, src, \
+                     rhs, T(dxinv), T(lambda), T(alpha), T(beta), T(fr.c1), T(fr.c2))
+  if (lap && zero_src) TWO_LAUNCH(true, true);
+  else if (lap) TWO_LAUNCH(true, false);
+  else if (zero_src) TWO_LAUNCH(false, true);
+  else TWO_LAUNCH(false, false);
+#undef TWO_LAUNCH
+  hip_check(hipGetLastError(), "k_gsrb_zmarch2");
+  prof_end(L.ctx, ev, KC_GSRB, (zero_src ? 16.0 : 24.0) * sizeof(T) / 8.0 * L.valid_cells, 2.0 * L.valid_cells);
+}
+// Tiles: 24 x 24 columns (512 threads, 126 registers in FP64, two workgroups a CU) read and compute
+// 32 x 32 / 24 x 24 = 1.8 times their cells; the march is bound by issue and LDS, not by memory
+// (400^3 FP64: 437 us, 303 us from zero, 3.5 and 3.4 TB/s of its 24 and 16 bytes a cell, where two launches
+// of the best marching tiles take 771 and 634; 1024-thread tiles of 64 x 20 and 32 x 43: 457 and 440).
+// FP32 levels above 12 million cells take 40 x 24 (768 threads: 248 and 174 us, 24 x 24 278 and 189, two
+// launches 433 and 366).  Chunks by size, so that the columns fill the chip: 12 planes (128 x 144 x
+// 128 FP64: 33 and 24 us, two launches 32 and 29), 16 (160^3: 42 and 30, two launches 48 and 45),
+// 32 (256^3: 129 and 89, two launches 210 and 176).
+template <class T>
+void gsrb_two(const DeviceLayout& L, const FaceRules& fr, T* dst, const T* src, const T* rhs, double dx, double alpha,
+              double beta, bool zero_src) {
+  if (dst == src || dst == rhs) throw std::runtime_error("gsrb_two: dst must be a separate field");
+  check_pair_pointer(dst, "gsrb_two");
+  check_pair_pointer(src, "gsrb_two");
+  check_pair_pointer(rhs, "gsrb_two");
+  const int kc = L.valid_cells < (3LL << 20) ? 12 : L.valid_cells < (12LL << 20) ? 16 : 32;
+  if constexpr (sizeof(T) == 4) {
+    if (L.valid_cells >= (12LL << 20)) {
+      launch_two<T, 40, 24, 768>(L, fr, dst, src, rhs, dx, alpha, beta, kc, zero_src);
+      return;
+    }
+  }
+  launch_two<T, 24, 24, 512>(L, fr, dst, src, rhs, dx, alpha, beta, kc, zero_src);
+}
+template void gsrb_two<double>(const DeviceLayout&, const FaceRules&, double*, const double*, const double*, double,
+                               double, double, bool);
+template void gsrb_two<float>(const DeviceLayout&, const FaceRules&, float*, const float*, const float*, double,
+                              double, double, bool);
 
 // Times every tile shape (and z-chunk lengths) of the one-launch relaxation on
 // this level's own fields and returns the fastest as {shape, kc}; times[] (if

@@ -80,6 +80,10 @@ struct FaceRules {
 template <class T>
 void gsrb_fused(const DeviceLayout& L, const FaceRules& fr, T* dst, const T* src, const T* rhs, double dx,
                 double alpha, double beta, int shape = -1, int kc = 0, bool zero_src = false);
+// Two such iterations in one launch: bitwise gsrb_fused twice
+template <class T>
+void gsrb_two(const DeviceLayout& L, const FaceRules& fr, T* dst, const T* src, const T* rhs, double dx,
+              double alpha, double beta, bool zero_src);
 // Autotuner of the one-launch relaxation: times every tile shape with z-chunk
 // lengths {auto, 8, 16, 32} on the given fields, returns the fastest {shape, kc};
 // times (kFusedShapeCount x 4 entries, ms per launch) receives all timings when not null.
