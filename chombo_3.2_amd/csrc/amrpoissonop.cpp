@@ -487,6 +487,15 @@ void AMRPoissonOp<Real>::relaxFromZero(T& e, const T& r, int n) {
     relaxBlocks(e, r, n, true, nullptr, nullptr);
     return;
   }
+  if (m_vc && n > 0 && m_fused && m_ctx->fused_relax && m_relaxMode == 1 && e.nc == 1 && m_vcShape < 0 &&
+      vc::marches<Real>(*m_lay, *m_vc)) {
+    need(e.lay, m_lay, "relaxFromZero"); need(r.lay, m_lay, "relaxFromZero");
+    if (!m_relaxTmp.isDefined()) m_relaxTmp.define(m_lay);
+    vc::gsrb_fused<Real>(*m_lay, m_faces, *m_vc, m_relaxTmp.d, e.d, r.d, m_dx, m_alpha, m_beta, m_vcShape, true);
+    std::swap(e.d, m_relaxTmp.d);
+    relax(e, r, n - 1);
+    return;
+  }
   if (n > 1 && e.own && pairMarches()) {
     relaxPairs(e, r, n / 2, true);
     if (n % 2) relax(e, r, 1);

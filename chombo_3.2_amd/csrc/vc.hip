@@ -14,6 +14,7 @@
 #include "fused.hpp"
 #include "ops.hpp"
 #include "vc.hpp"
+#include "vczmarch.hpp"
 
 namespace amrmg {
 
@@ -353,15 +354,6 @@ __global__ void __launch_bounds__(256) k_vc_avg_faces(const DBox* __restrict__ c
 // the cell's six faces from global memory, two steps ahead of their use.
 // ---------------------------------------------------------------------------
 template <class T>
-struct VCFused {
-  const T* a;
-  const T* b0;
-  const T* b1;
-  const T* b2;
-  long long foff[3];  // face index of the rectangle's low corner, per direction
-  int fsy[3], fsz[3];
-};
-template <class T>
 struct VCCell {  // operands of one update
   T r, a, b0m, b0p, b1m, b1p, b2m, b2p;
 };
@@ -554,9 +546,23 @@ __global__ void __launch_bounds__(NT) k_vc_gsrb_fused(ops::FusedArgs a, VCFused<
   ops::lds_barrier();
   store(k1 - 1);
 }
-// tile shapes of the one-launch VC relaxation {FX, FY, NT}
+template <class T, int FX, int FY, int NT, bool ZSRC>
+__global__ void __launch_bounds__(NT) k_vc_zmarch(ops::FusedArgs a, VCFused<T> v, T* __restrict__ dst,
+                                                  const T* __restrict__ src, const T* __restrict__ rhs, T dxinv,
+                                                  T scale, T alpha, T beta, T c1, T c2) {
+  const int w = ops::xcd_contiguous_block();
+  if (w >= a.nwork) return;
+  vc_zmarch_body<T, FX, FY, NT, ZSRC>(a, v, w, dst, src, rhs, dxinv, scale, alpha, beta, c1, c2);
+}
+// tile shapes of k_vc_gsrb_fused {FX, FY, NT}, for those who ask for one
 constexpr int kVCShapes[][3] = {{64, 8, 256}, {32, 8, 256}, {64, 4, 256}, {64, 16, 512}};
 constexpr int kVCShapeCount = 4;
+// The automatic choice: k_vc_zmarch, 32 x 10 columns in 256 threads (172 to 196 registers in FP64: two
+// workgroups a CU) and chunks of 8 planes, 4 where those are fewer than 512.  The relaxations of a 3-level
+// 128^3 solve (2 to 8 million cells): 12.9 ms, where k_vc_gsrb_fused's best tiles (64 x 4, 32 x 8
+// where narrower) took 20.6; 32 x 24 in 512 threads 20, chunks of 16 and 24 planes 13.4 and 15.1,
+// registers held to 168 (spilled) 17.4.
+constexpr int kVCColX = 32, kVCColY = 10, kVCColT = 256;
 
 #define VC_LAUNCH(L, kind, bytes, units, kernel, grid, ...)                                \
   do {                                                                                     \
@@ -606,17 +612,28 @@ void gsrb(const DeviceLayout& L, const VCCoefs<T>& C, T* phi, const T* rhs, int 
             args(C), phi, rhs, color, T(dxinv), T(alpha), T(beta));
 }
 template <class T>
+bool marches(const DeviceLayout& L, const VCCoefs<T>& C) {
+  if (!L.merged) return false;
+  // a plane of cells or faces is addressed with 32-bit byte offsets
+  bool ok = (long long)L.h_boxes[L.nbox].sz * (long long)sizeof(T) < (1LL << 31);
+  for (int d = 0; d < 3; d++) {
+    const DBox& f = C.h_fbox[d][L.nbox];
+    ok = ok && ((long long)f.sz + f.sy) * (long long)sizeof(T) < (1LL << 31);
+  }
+  return ok;
+}
+template <class T>
 void gsrb_fused(const DeviceLayout& L, const ops::FaceRules& fr, const VCCoefs<T>& C, T* dst, const T* src,
-                const T* rhs, double dx, double alpha, double beta, int shape) {
+                const T* rhs, double dx, double alpha, double beta, int shape, bool zero_src) {
   need_coefs(L, C, "vc::gsrb_fused");
   if (!L.merged) throw std::runtime_error("vc::gsrb_fused: level is not stored merged");
   if (dst == src || dst == rhs) throw std::runtime_error("vc::gsrb_fused: dst must be a separate field");
   const DBox& R = L.h_boxes[L.nbox];
-  // automatic: 64-wide columns where the level is that wide, 4 rows in FP64 (fewer
-  // registers: more waves in flight), 8 in FP32; 32 x 8 on narrower levels
-  if (shape < 0) shape = (R.hi[0] - R.lo[0] + 1 >= 64) ? (sizeof(T) == 8 ? 2 : 0) : 1;
   if (shape >= kVCShapeCount) throw std::runtime_error("vc::gsrb_fused: bad tile shape");
-  const int FX = kVCShapes[shape][0], FY = kVCShapes[shape][1];
+  const bool march = shape < 0 && marches<T>(L, C);
+  if (!march && shape < 0) shape = 2;
+  if (zero_src && !march) throw std::runtime_error("vc::gsrb_fused: this tile shape reads the old values");
+  const int FX = march ? kVCColX : kVCShapes[shape][0], FY = march ? kVCColY : kVCShapes[shape][1];
   ops::FusedArgs a;
   for (int q = 0; q < 3; q++) {
     a.lo[q] = R.lo[q];
@@ -630,12 +647,19 @@ void gsrb_fused(const DeviceLayout& L, const ops::FaceRules& fr, const VCCoefs<T
   a.off = R.off;
   a.sy = R.sy;
   a.sz = R.sz;
+  if (march) {
+    ops::check_pair_rows(a);
+    ops::check_pair_pointer(src, "vc::gsrb_fused");
+    ops::check_pair_pointer(dst, "vc::gsrb_fused");
+    ops::check_pair_pointer(rhs, "vc::gsrb_fused");
+    ops::check_pair_pointer((const T*)C.a.d, "vc::gsrb_fused");
+  }
   a.zsrc = 0;
   a.ntx = (R.hi[0] - R.lo[0] + 1 + FX - 1) / FX;
   a.nty = (R.hi[1] - R.lo[1] + 1 + FY - 1) / FY;
   const int nz = R.hi[2] - R.lo[2] + 1;
-  int kc = 32;
-  while (kc > 4 && (long long)a.ntx * a.nty * ((nz + kc - 1) / kc) < 2048) kc >>= 1;
+  int kc = march ? 8 : 32;
+  while (kc > 4 && (long long)a.ntx * a.nty * ((nz + kc - 1) / kc) < (march ? 512 : 2048)) kc >>= 1;
   a.kc = kc;
   const long long nwork = (long long)a.ntx * a.nty * ((nz + kc - 1) / kc);
   if (nwork > INT32_MAX - 8) throw std::runtime_error("vc::gsrb_fused: level too large");
@@ -661,13 +685,23 @@ void gsrb_fused(const DeviceLayout& L, const ops::FaceRules& fr, const VCCoefs<T
     hipLaunchKernelGGL((k_vc_gsrb_fused<T, X, Y, NT>), dim3(grid), dim3(NT), 0, L.ctx->stream, a, v, dst, src, rhs, \
                        T(dxinv), T(scale), T(alpha), T(beta), T(fr.c1), T(fr.c2));                              \
     break;
-  switch (shape) {
-    VC_FUSED_CASE(0, 64, 8, 256)
-    VC_FUSED_CASE(1, 32, 8, 256)
-    VC_FUSED_CASE(2, 64, 4, 256)
-    VC_FUSED_CASE(3, 64, 16, 512)
+#define VC_MARCH(Z)                                                                                              \
+  hipLaunchKernelGGL((k_vc_zmarch<T, kVCColX, kVCColY, kVCColT, Z>), dim3(grid), dim3(kVCColT), 0, L.ctx->stream, a, \
+                     v, dst, src, rhs, T(dxinv), T(scale), T(alpha), T(beta), T(fr.c1), T(fr.c2))
+  if (march && zero_src) {
+    VC_MARCH(true);
+  } else if (march) {
+    VC_MARCH(false);
+  } else {
+    switch (shape) {
+      VC_FUSED_CASE(0, 64, 8, 256)
+      VC_FUSED_CASE(1, 32, 8, 256)
+      VC_FUSED_CASE(2, 64, 4, 256)
+      VC_FUSED_CASE(3, 64, 16, 512)
+    }
   }
 #undef VC_FUSED_CASE
+#undef VC_MARCH
   hip_check(hipGetLastError(), "k_vc_gsrb_fused");
   profile_end(L.ctx, ev, KC_GSRB, bytes, units);
 }
@@ -822,8 +856,9 @@ void narrow(const VCCoefs<double>& src, VCCoefs<float>& dst) {
 
 #define VC_INST(T)                                                                                                  \
   template void gsrb<T>(const DeviceLayout&, const VCCoefs<T>&, T*, const T*, int, double, double, double);        \
+  template bool marches<T>(const DeviceLayout&, const VCCoefs<T>&);                                               \
   template void gsrb_fused<T>(const DeviceLayout&, const ops::FaceRules&, const VCCoefs<T>&, T*, const T*,          \
-                              const T*, double, double, double, int);                                               \
+                              const T*, double, double, double, int, bool);                                         \
   template void apply<T>(const DeviceLayout&, const VCCoefs<T>&, T*, const T*, double, double, double);            \
   template void residual<T>(const DeviceLayout&, const VCCoefs<T>&, T*, const T*, const T*, double, double, double); \
   template void restrict_res<T>(const DeviceLayout&, const DeviceLayout&, const VCCoefs<T>&, T*, const T*,          \

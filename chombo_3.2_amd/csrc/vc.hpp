@@ -52,12 +52,16 @@ namespace vc {
 template <class T>
 void gsrb(const DeviceLayout& L, const VCCoefs<T>& C, T* phi, const T* rhs, int color, double dx, double alpha,
           double beta);
+// whether gsrb_fused's automatic shape on this level is the z march, which takes zero_src
+template <class T>
+bool marches(const DeviceLayout& L, const VCCoefs<T>& C);
 // One GSRB iteration (red, refresh, black) of a merged level in one launch:
 // dst <- relaxed src, bitwise equal to the ghost refresh + gsrb(0) + ghost refresh
-// + gsrb(1) sequence.  shape: tile shape (-1 automatic, 0..3).
+// + gsrb(1) sequence.  shape: tile shape (-1 automatic, 0..3); zero_src: src is known to be zero and
+// not read (where marches() holds).
 template <class T>
 void gsrb_fused(const DeviceLayout& L, const ops::FaceRules& fr, const VCCoefs<T>& C, T* dst, const T* src,
-                const T* rhs, double dx, double alpha, double beta, int shape = -1);
+                const T* rhs, double dx, double alpha, double beta, int shape = -1, bool zero_src = false);
 // VCCOMPUTEOP (VCAMRPoissonOpF.ChF:197-265)
 template <class T>
 void apply(const DeviceLayout& L, const VCCoefs<T>& C, T* lofphi, const T* phi, double dx, double alpha,

@@ -257,11 +257,16 @@ __device__ __forceinline__ void zmarch_body(const FusedArgs& a, int w, T* __rest
   step(I1{}, F{}, k0 - 1);
   for (int kb = k0 - 2; kb + 2 < k1; kb += 6) {
     step(I2{}, Tr{}, kb + 2);
-    if (kb + 3 < k1) step(I3{}, Tr{}, kb + 3);
-    if (kb + 4 < k1) step(I4{}, Tr{}, kb + 4);
-    if (kb + 5 < k1) step(I5{}, Tr{}, kb + 5);
-    if (kb + 6 < k1) step(I0{}, Tr{}, kb + 6);
-    if (kb + 7 < k1) step(I1{}, Tr{}, kb + 7);
+    if (kb + 3 >= k1) break;
+    step(I3{}, Tr{}, kb + 3);
+    if (kb + 4 >= k1) break;
+    step(I4{}, Tr{}, kb + 4);
+    if (kb + 5 >= k1) break;
+    step(I5{}, Tr{}, kb + 5);
+    if (kb + 6 >= k1) break;
+    step(I0{}, Tr{}, kb + 6);
+    if (kb + 7 >= k1) break;
+    step(I1{}, Tr{}, kb + 7);
   }
 }
 
@@ -497,11 +502,16 @@ __device__ __forceinline__ void zmarch4_body(const FusedArgs& a, int w, T* __res
   step(I1{}, F{}, k0 - 1);
   for (int kb = k0 - 2; kb + 2 < k1; kb += 6) {
     step(I2{}, Tr{}, kb + 2);
-    if (kb + 3 < k1) step(I3{}, Tr{}, kb + 3);
-    if (kb + 4 < k1) step(I4{}, Tr{}, kb + 4);
-    if (kb + 5 < k1) step(I5{}, Tr{}, kb + 5);
-    if (kb + 6 < k1) step(I0{}, Tr{}, kb + 6);
-    if (kb + 7 < k1) step(I1{}, Tr{}, kb + 7);
+    if (kb + 3 >= k1) break;
+    step(I3{}, Tr{}, kb + 3);
+    if (kb + 4 >= k1) break;
+    step(I4{}, Tr{}, kb + 4);
+    if (kb + 5 >= k1) break;
+    step(I5{}, Tr{}, kb + 5);
+    if (kb + 6 >= k1) break;
+    step(I0{}, Tr{}, kb + 6);
+    if (kb + 7 >= k1) break;
+    step(I1{}, Tr{}, kb + 7);
   }
 }
 

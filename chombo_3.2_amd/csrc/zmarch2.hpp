@@ -186,11 +186,16 @@ __device__ __forceinline__ void zmarch2_body(const FusedArgs& a, int w, T* __res
   ZM2_STEP(5, 3, k0 - 1);
   for (int kb = k0; kb < k1; kb += 6) {
     ZM2_STEP(0, 4, kb);
-    if (kb + 1 < k1) ZM2_STEP(1, 4, kb + 1);
-    if (kb + 2 < k1) ZM2_STEP(2, 4, kb + 2);
-    if (kb + 3 < k1) ZM2_STEP(3, 4, kb + 3);
-    if (kb + 4 < k1) ZM2_STEP(4, 4, kb + 4);
-    if (kb + 5 < k1) ZM2_STEP(5, 4, kb + 5);
+    if (kb + 1 >= k1) break;
+    ZM2_STEP(1, 4, kb + 1);
+    if (kb + 2 >= k1) break;
+    ZM2_STEP(2, 4, kb + 2);
+    if (kb + 3 >= k1) break;
+    ZM2_STEP(3, 4, kb + 3);
+    if (kb + 4 >= k1) break;
+    ZM2_STEP(4, 4, kb + 4);
+    if (kb + 5 >= k1) break;
+    ZM2_STEP(5, 4, kb + 5);
   }
 #undef ZM2_STEP
 }
