@@ -217,8 +217,9 @@ void block_visit(const DeviceLayout& L, const FaceRules& fr, const DeviceLayout*
   const bool lap = (alpha == 0.0 && beta == 1.0);
   const double lambda = lap ? -1.0 / sum_b : -1.0 / (alpha - beta * sum_b);
   const T* s = zero_src ? nullptr : src;
-  // algorithmic bytes of the relaxation, as gsrb_fused counts them
-  const double bytes = ((zero_src ? 16.0 : 24.0) + 24.0 * (sweeps - 1)) * sizeof(T) / 8.0 * L.valid_cells;
+  // algorithmic bytes of the visit: read phi (not when it is known zero), read rhs, write phi; the
+  // coarse field
+  const double bytes = ((zero_src ? 16.0 : 24.0) + (coarse || resc ? 1.0 : 0.0)) * sizeof(T) / 8.0 * L.valid_cells;
   hipEvent_t ev = profile_begin(L.ctx, KC_GSRB);
 #define BLOCK_LAUNCH(LAPV, NS, RESTV)                                                                            \
   hipLaunchKernelGGL((k_block_visit<T, LAPV, kBX, kBY, kBZ, NS, RESTV, kBT>), dim3(grid), dim3(kBT), 0,         \

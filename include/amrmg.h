@@ -188,16 +188,18 @@ int amrmg_bottom_solve_device(amrmg_solver* s, double* corr, const double* res, 
 int amrmg_solver_set_bottom_params(amrmg_solver* s, const int* ip, const double* rp);
 
 /* Autotuner of the one-launch relaxation: on every level that uses it, times its
-   10 tile shapes (columns 64x8, 32x8, 64x4, 32x16, 128x4, 64x16 of 256 threads;
-   32x16, 64x16 of 512; 64x32, 128x8 of 1024) x z-chunk lengths {auto, 8, 16, 32}
-   on the solver's own fields and keeps the fastest for later solves (results are
-   bitwise the same for every choice).  Writes up to cap records of 46 doubles:
+   26 tile shapes x z-chunk lengths {auto, 8, 16, 32}
+   on the solver's own fields and keeps the fastest for later single iterations (results are
+   bitwise the same for every choice; pairs of iterations and the visits of levels of up to a
+   million cells run in kernels of their own, which are not tuned).  Writes up to cap records of
+   110 doubles:
    {0 AMR level / 1 multigrid depth, index, valid cells, chosen shape, chosen
    z-chunk, its ms per iteration, then ms of each shape x chunk}; *nrec = number
    of tuned levels. */
 int amrmg_solver_tune_relax(amrmg_solver* s, double* table, int cap, int* nrec);
-/* Forces tile shape (0..12) and z-chunk (0 = automatic) of the one-launch
-   relaxation on every level. */
+/* Forces tile shape (0..25) and z-chunk (0 = automatic) of the one-launch
+   relaxation on every level: each iteration is then a launch of that shape, also where two
+   iterations or a whole visit would run as one (results are bitwise the same). */
 int amrmg_solver_set_relax_shape(amrmg_solver* s, int shape, int kc);
 /* AMRPoissonOp::s_relaxMode (AMRPoissonOp.cpp:31, 600-632) for every operator of the
    solver: 0 looseGSRB (AMRPoissonOp.cpp:1333-1413), 1 levelGSRB (default), 2
@@ -208,7 +210,7 @@ int amrmg_solver_set_relax_shape(amrmg_solver* s, int shape, int kc);
    the host-driven BiCGStab. */
 int amrmg_solver_set_relax_mode(amrmg_solver* s, int mode);
 /* Tile shape of the one-launch variable-coefficient relaxation on every multigrid
-   depth: -1 automatic, 0 64x8, 1 32x8, 2 64x4 (256 threads), 3 64x16 (512
+   depth: -1 automatic (a z march), 0 64x8, 1 32x8, 2 64x4 (256 threads), 3 64x16 (512
    threads); results are bitwise the same for every choice.  No counterpart in the
    reference (its GSRBHELMHOLTZVC runs per box and colour). */
 int amrmg_solver_set_vc_relax_shape(amrmg_solver* s, int shape);
