@@ -387,15 +387,17 @@ __device__ __forceinline__ bool tile_cell(const DBox* __restrict__ boxes, const 
   return i <= b.hi[0] && j <= b.hi[1] && k <= b.hi[2];
 }
 
-#define LAUNCH_PU(kind, bytes, units, kernel, grid, ...)                                 \
+#define LAUNCH_TU(threads, kind, bytes, units, kernel, grid, ...)                        \
   do {                                                                                   \
     if ((grid) > 0) {                                                                    \
       hipEvent_t ev_ = prof_begin(L.ctx, kind);                                          \
-      hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, L.ctx->stream, __VA_ARGS__);   \
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, L.ctx->stream, __VA_ARGS__); \
       hip_check(hipGetLastError(), #kernel);                                             \
       prof_end(L.ctx, ev_, kind, bytes, units);                                          \
     }                                                                                    \
   } while (0)
+#define LAUNCH_PU(kind, bytes, units, kernel, grid, ...) LAUNCH_TU(256, kind, bytes, units, kernel, grid, __VA_ARGS__)
+#define LAUNCH_T(threads, kind, bytes, kernel, grid, ...) LAUNCH_TU(threads, kind, bytes, 0.0, kernel, grid, __VA_ARGS__)
 #define LAUNCH_P(kind, bytes, kernel, grid, ...) LAUNCH_PU(kind, bytes, 0.0, kernel, grid, __VA_ARGS__)
 #define LAUNCH(kernel, grid, ...) LAUNCH_P(KC_BLAS, 0.0, kernel, grid, __VA_ARGS__)
 
@@ -979,35 +981,96 @@ __global__ void __launch_bounds__(256) k_apply_residual(const DBox* __restrict__
   const T lap = (phi[c + 1] + phi[c - 1] + phi[c + sy] + phi[c - sy] + phi[c + sz] + phi[c - sz] - T(6.0) * p) * dxinv;
   res[c] = apply_axby(alpha * p + beta * lap, rhs[c]);
 }
-template <class T>
-__global__ void __launch_bounds__(256) k_apply_residual_z(const DBox* __restrict__ boxes,
-                                                          const Tile* __restrict__ ctiles, int nct, int kz,
-                                                          T* __restrict__ res, const T* __restrict__ phi,
-                                                          const T* __restrict__ rhs, T dxinv, T alpha, T beta) {
+// The residual of a merged level over its 64 x 4 column tiles, marching in z with x pairs: a lane
+// holds its pair's planes below and above in registers and loads what the next plane takes (the pair two
+// planes up, rhs, the pairs of the rows beside and the two far x cells) a plane ahead.  Bound by
+// memory; a lane per cell with each plane's loads waited for in turn reached 3.9 TB/s of the 24
+// bytes a cell (337 us a launch on average in the 3-level 256^3 solve, 150 us with AXBY), this 4.5 TB/s
+// (289 and 135 us); the rest is the tiles' halo rows and planes.
+// AXBY: AMRResidual's expression, else OPERATORLAPRES.
+// nrm (optional): the max-norm of what is written is folded into *nrm as k_maxnorm
+// folds it (per-block max, then an atomic max of the non-negative bit pattern, skipped
+// when the block's max does not exceed the value already there)
+template <class T, bool AXBY>
+__global__ void __launch_bounds__(128) k_residual_z(const DBox* __restrict__ boxes, const Tile* __restrict__ ctiles,
+                                                    int nct, int kz, T* res, const T* __restrict__ phi, const T* rhs,
+                                                    T dxinv, T alpha, T beta, double* nrm) {
+  using P2 = Pair<T>;
   const int w = xcd_contiguous_block();
-  if (w >= nct) return;
+  if (w >= nct) return;  // uniform over the block
   const Tile t = ctiles[w];
   const DBox b = boxes[t.box];
-  const int i = t.i0 + (threadIdx.x & 63), j = t.j0 + (threadIdx.x >> 6);
-  if (i > b.hi[0] || j > b.hi[1]) return;
-  const int kend = min(t.k0 + kz - 1, b.hi[2]);
-  const long long sy = b.sy, sz = b.sz;
-  long long c = cidx(b, i, j, t.k0);
-  T pm = phi[c - sz], p = phi[c];
-  for (int k = t.k0; k <= kend; k++, c += sz) {
-    const T pz = phi[c + sz];
-    const T lap = (phi[c + 1] + phi[c - 1] + phi[c + sy] + phi[c - sy] + pz + pm - T(6.0) * p) * dxinv;
-    res[c] = apply_axby(alpha * p + beta * lap, rhs[c]);
-    pm = p;
-    p = pz;
+  const int i = t.i0 + 2 * (threadIdx.x & 31), j = t.j0 + (threadIdx.x >> 5);
+  double v = 0.0;
+  if (i <= b.hi[0] && j <= b.hi[1]) {
+    const bool two = i + 1 <= b.hi[0];  // else the pair's second cell is the ghost cell hi[0] + 1
+    const int kend = min(t.k0 + kz - 1, b.hi[2]);
+    const long long sy = b.sy, sz = b.sz;
+    long long c = cidx(b, i, j, t.k0);
+    auto pair = [](const T* f, long long q) { return *reinterpret_cast<const P2*>(f + q); };
+    P2 pm = pair(phi, c - sz), p = pair(phi, c), pz = pair(phi, c + sz);
+    P2 r = pair(rhs, c), ym = pair(phi, c - sy), yp = pair(phi, c + sy);
+    T xl = phi[c - 1], xr = phi[c + 2];
+    for (int k = t.k0; k <= kend; k++, c += sz) {
+      // the next plane's operands (the last plane loads its own again)
+      const long long n = k < kend ? c + sz : c;
+      const P2 pzn = pair(phi, n + sz), rn = pair(rhs, n), ymn = pair(phi, n - sy), ypn = pair(phi, n + sy);
+      const T xln = phi[n - 1], xrn = phi[n + 2];
+      const T lap0 = (p.y + xl + yp.x + ym.x + pz.x + pm.x - T(6.0) * p.x) * dxinv;
+      const T lap1 = (xr + p.x + yp.y + ym.y + pz.y + pm.y - T(6.0) * p.y) * dxinv;
+      P2 o;
+      if (AXBY) {
+        o.x = apply_axby(alpha * p.x + beta * lap0, r.x);
+        o.y = apply_axby(alpha * p.y + beta * lap1, r.y);
+      } else {
+        o.x = -(alpha * p.x) - beta * lap0 + r.x;
+        o.y = -(alpha * p.y) - beta * lap1 + r.y;
+      }
+      v = fmax(v, fabs((double)o.x));
+      if (two) {
+        *reinterpret_cast<P2*>(res + c) = o;
+        v = fmax(v, fabs((double)o.y));
+      } else {
+        res[c] = o.x;
+      }
+      pm = p;
+      p = pz;
+      pz = pzn;
+      r = rn;
+      ym = ymn;
+      yp = ypn;
+      xl = xln;
+      xr = xrn;
+    }
   }
+  if (nrm) {  // uniform over the launch
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    __shared__ double sm[2];
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const double m = fmax(sm[0], sm[1]);
+      if (m > 0.0 && m > *(volatile double*)nrm)
+        atomicMax((unsigned long long*)nrm, (unsigned long long)__double_as_longlong(m));
+    }
+  }
+}
+// whether k_residual_z applies: a merged level whose pairs are aligned in the fields
+template <class T>
+static bool residual_z_ok(const DeviceLayout& L, const T* res, const T* phi, const T* rhs) {
+  if (!(L.merged && L.nctiles > 0)) return false;
+  const DBox& R = L.h_boxes[L.nbox];
+  const uintptr_t m = reinterpret_cast<uintptr_t>(res) | reinterpret_cast<uintptr_t>(phi) |
+                      reinterpret_cast<uintptr_t>(rhs);
+  return (R.off + 1) % 2 == 0 && R.sy % 2 == 0 && R.sz % 2 == 0 && m % (2 * sizeof(T)) == 0;
 }
 template <class T>
 void apply_residual(const DeviceLayout& L, T* res, const T* phi, const T* rhs, double dx, double alpha, double beta) {
   double dxinv = 1.0 / (dx * dx);
-  if (L.merged && L.nctiles > 0) {
-    LAUNCH_P(KC_APPLY, 3.0 * sizeof(T) * L.valid_cells, k_apply_residual_z<T>, (L.nctiles + 7) / 8 * 8, L.d_boxes,
-             L.d_ctiles, L.nctiles, DeviceLayout::kColumnPlanes, res, phi, rhs, T(dxinv), T(alpha), T(beta));
+  if (residual_z_ok(L, res, phi, rhs)) {
+    LAUNCH_T(128, KC_APPLY, 3.0 * sizeof(T) * L.valid_cells, (k_residual_z<T, true>), (L.nctiles + 7) / 8 * 8, L.d_boxes,
+             L.d_ctiles, L.nctiles, DeviceLayout::kColumnPlanes, res, phi, rhs, T(dxinv), T(alpha), T(beta),
+             (double*)nullptr);
     return;
   }
   LAUNCH_P(KC_APPLY, 3.0 * sizeof(T) * L.valid_cells, k_apply_residual<T>, L.ntiles, L.d_boxes, L.d_tiles, geom(L), res,
@@ -1028,52 +1091,11 @@ __global__ void __launch_bounds__(256) k_residual(const DBox* __restrict__ boxes
   const T lap = (phi[c + 1] + phi[c - 1] + phi[c + sy] + phi[c - sy] + phi[c + sz] + phi[c - sz] - T(6.0) * p) * dxinv;
   res[c] = -(alpha * p) - beta * lap + rhs[c];
 }
-// the same over a merged level's column tiles, marching in z (as k_apply_z).
-// nrm (optional): the max-norm of what is written is folded into *nrm as k_maxnorm
-// folds it (per-block max, then an atomic max of the non-negative bit pattern, skipped
-// when the block's max does not exceed the value already there)
-template <class T>
-__global__ void __launch_bounds__(256) k_residual_z(const DBox* __restrict__ boxes, const Tile* __restrict__ ctiles,
-                                                    int nct, int kz, T* res, const T* __restrict__ phi, const T* rhs,
-                                                    T dxinv, T alpha, T beta, double* nrm) {
-  const int w = xcd_contiguous_block();
-  if (w >= nct) return;  // uniform over the block
-  const Tile t = ctiles[w];
-  const DBox b = boxes[t.box];
-  const int i = t.i0 + (threadIdx.x & 63), j = t.j0 + (threadIdx.x >> 6);
-  double v = 0.0;
-  if (i <= b.hi[0] && j <= b.hi[1]) {
-    const int kend = min(t.k0 + kz - 1, b.hi[2]);
-    const long long sy = b.sy, sz = b.sz;
-    long long c = cidx(b, i, j, t.k0);
-    T pm = phi[c - sz], p = phi[c];
-    for (int k = t.k0; k <= kend; k++, c += sz) {
-      const T pz = phi[c + sz];
-      const T lap = (phi[c + 1] + phi[c - 1] + phi[c + sy] + phi[c - sy] + pz + pm - T(6.0) * p) * dxinv;
-      const T r = -(alpha * p) - beta * lap + rhs[c];
-      res[c] = r;
-      v = fmax(v, fabs((double)r));
-      pm = p;
-      p = pz;
-    }
-  }
-  if (nrm) {  // uniform over the launch
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    __shared__ double sm[4];
-    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const double m = fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3]));
-      if (m > 0.0 && m > *(volatile double*)nrm)
-        atomicMax((unsigned long long*)nrm, (unsigned long long)__double_as_longlong(m));
-    }
-  }
-}
 template <class T>
 void residual(const DeviceLayout& L, T* res, const T* phi, const T* rhs, double dx, double alpha, double beta) {
   double dxinv = 1.0 / (dx * dx);
-  if (L.merged && L.nctiles > 0) {
-    LAUNCH_P(KC_RESIDUAL, 3.0 * sizeof(T) * L.valid_cells, k_residual_z<T>, (L.nctiles + 7) / 8 * 8, L.d_boxes,
+  if (residual_z_ok(L, res, phi, rhs)) {
+    LAUNCH_T(128, KC_RESIDUAL, 3.0 * sizeof(T) * L.valid_cells, (k_residual_z<T, false>), (L.nctiles + 7) / 8 * 8, L.d_boxes,
              L.d_ctiles, L.nctiles, DeviceLayout::kColumnPlanes, res, phi, rhs, T(dxinv), T(alpha), T(beta),
              (double*)nullptr);
     return;
@@ -1532,14 +1554,14 @@ void maxnorm_async(const DeviceLayout& L, const T* x, int slot, int accumulate) 
 template <class T>
 void residual_norm(const DeviceLayout& L, T* res, const T* phi, const T* rhs, double dx, double alpha, double beta,
                    int slot, int accumulate) {
-  if (!(L.merged && L.nctiles > 0)) {
+  if (!residual_z_ok(L, res, phi, rhs)) {
     residual<T>(L, res, phi, rhs, dx, alpha, beta);
     maxnorm_async<T>(L, res, slot, accumulate);
     return;
   }
   if (!accumulate) LAUNCH(k_zero_scalar, 1, L.ctx->d_scalars, slot);
   const double dxinv = 1.0 / (dx * dx);
-  LAUNCH_P(KC_RESIDUAL, 3.0 * sizeof(T) * L.valid_cells, k_residual_z<T>, (L.nctiles + 7) / 8 * 8, L.d_boxes,
+  LAUNCH_T(128, KC_RESIDUAL, 3.0 * sizeof(T) * L.valid_cells, (k_residual_z<T, false>), (L.nctiles + 7) / 8 * 8, L.d_boxes,
            L.d_ctiles, L.nctiles, DeviceLayout::kColumnPlanes, res, phi, rhs, T(dxinv), T(alpha), T(beta),
            L.ctx->d_scalars + slot);
 }
