@@ -9,7 +9,7 @@ GSRB sweeps and a BiCGStab bottom solve.
 
 Prints one JSON line.  value = Mcell-relax/s (cells x red-black GSRB iterations
 over every level relaxed, per second of solve wall time).  roofline = the GSRB
-kernel's algorithmic bytes (24 B per cell-relax in FP64) over its HIP-event time
+kernels' algorithmic bytes (24 B per cell and launch in FP64, 16 B from zero) over their HIP-event time
 inside the timed region, against 8 TB/s HBM.  cpu_baseline = the oracle (a C
 restatement of the reference's FP64 path, OpenMP over boxes) built for the host CPU
 and timed on one full solve of the same workload (setup excluded).
@@ -130,7 +130,7 @@ def summarize_pmc(fetch_csv, write_csv, fetch_json, copy_bytes, out_path):
         rows = sorted(csv.DictReader(open(path)), key=lambda r: int(r["Dispatch_Id"]))
         first_cp = min(q for q, r in enumerate(rows) if "k_copy_probe" in r["Kernel_Name"])
         gs = [float(r["Counter_Value"]) * 1024.0 for r in rows[:first_cp]
-              if "k_gsrb_fused" in r["Kernel_Name"] or "k_gsrb_zmarch" in r["Kernel_Name"]]
+              if any(k in r["Kernel_Name"] for k in ("k_gsrb_fused", "k_gsrb_zmarch", "k_block_visit"))]
         cp = [float(r["Counter_Value"]) * 1024.0 for r in rows if "k_copy_probe" in r["Kernel_Name"]]
         if len(gs) < n:
             raise SystemExit(f"dispatch count mismatch: {len(gs)} relaxations before the calibration, {n} timed")
@@ -143,7 +143,7 @@ def summarize_pmc(fetch_csv, write_csv, fetch_json, copy_bytes, out_path):
     meas_total = sum(gf) * fscale + sum(gw) * wscale
     ratio = meas_total / alg_total
     d = {
-        "kernel": "GSRB relaxation class (k_gsrb_fused, k_gsrb_zmarch)",
+        "kernel": "GSRB relaxation class (k_gsrb_zmarch2, k_block_visit, k_gsrb_zmarch, k_gsrb_fused)",
         "fetch_scale": round(fscale, 4), "write_scale": round(wscale, 4),
         "copy_bytes": copy_bytes,
         "gsrb_dispatches": len(gf),
@@ -809,7 +809,7 @@ def main():
             "frac": round(achieved / PEAK_HBM_GBS, 4),
             "traffic": traffic,
             "traffic_over_algorithmic": ratio,
-            "kernel": "GSRB relaxation class: k_gsrb_fused / k_gsrb_zmarch (one red+black iteration of a whole level per launch)",
+            "kernel": "GSRB relaxation class: k_gsrb_zmarch2 / k_block_visit (two red+black iterations of a whole level per launch; bytes per launch, not per iteration), k_gsrb_zmarch / k_gsrb_fused (one)",
             "avg_launch_ms": round(avg_launch_ms, 5),
             "algorithmic_bytes_per_launch": round(bytes_per_launch, 1),
             "launches": prof["launches"],
