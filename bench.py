@@ -92,9 +92,10 @@ def summarize_trace(trace_csv, out_path, names, command):
             inst.setdefault(i, [0, 0.0])
             inst[i][0] += 1
             inst[i][1] += (e_ - s_) * 1e-6
-        # the roofline kernel: every one-launch relaxation (k_gsrb_fused, k_gsrb_zmarch, k_gsrb_zmarch4)
-        gs = [(e_ - s_) * 1e-6 for s_, e_, n in reg if re.match(r"k_gsrb_(fused|zmarch)", base(n))]
-        gline = (f"GSRB relaxation class (the roofline kernel): {len(gs)} launches, {sum(gs):.2f} ms, "
+        # the relaxation class: every launch of one iteration, of two, or of a small level's whole visit
+        gs = [(e_ - s_) * 1e-6 for s_, e_, n in reg
+              if re.match(r"k_gsrb_(fused|zmarch)|k_block_visit|k_vc_(gsrb_fused|zmarch)|k_batch_fused", base(n))]
+        gline = (f"Relaxation class: {len(gs)} launches, {sum(gs):.2f} ms, "
                  f"average {1000 * sum(gs) / len(gs):.1f} us per launch.") if gs else ""
         out += [f"## {title}", "", f"{len(reg)} dispatches, span {span:.2f} ms under the profiler, kernels busy "
                 f"{busy:.2f} ms.", ""] + ([gline, ""] if gline else []) + [
@@ -371,10 +372,14 @@ def vc_leg(args, ctx, h, rhs):
             s.solve()
         ctx.profile(["gsrb"])
         ctx.profile_reset()
+        if args.trace_marks:
+            ctx.copy_probe(4096, 1)
         t1 = time.perf_counter()
         for _ in range(args.steps):
             hist, info = s.solve()
         wall = time.perf_counter() - t1
+        if args.trace_marks:
+            ctx.copy_probe(4096, 1)
         prof = ctx.profile_read("gsrb")
         ctx.profile([])
         key = "fp64" if prec == 0 else "mixed"
@@ -477,10 +482,14 @@ def batch_leg(args, ctx):
         for _ in range(max(args.warmup, 1)):
             b.solve()  # the first V-cycle captures the graph
         # timed: profiler off, every V-cycle replayed from the captured HIP graph
+        if args.trace_marks:
+            ctx.copy_probe(4096, 1)
         t1 = time.perf_counter()
         for _ in range(args.steps):
             it, ex = b.solve()
         wall = (time.perf_counter() - t1) / args.steps
+        if args.trace_marks:
+            ctx.copy_probe(4096, 1)
         replays = b.set_graph(None)
         st = b.stats()
         phis = {q: b.get_phi(q) for q in phi_plain}
@@ -661,8 +670,8 @@ def main():
     ap.add_argument("--copy-mb", type=int, default=2048,
                     help="size of the plain copy kernel run after the timed region (0 = skip)")
     ap.add_argument("--trace-marks", action="store_true",
-                    help="launch a 4 KiB copy kernel before and after each timed region of the FP64 and mixed "
-                         "legs (region boundaries for --summarize-trace)")
+                    help="launch a 4 KiB copy kernel before and after each timed region of the FP64, mixed, "
+                         "variable-coefficient and batch legs (region boundaries for --summarize-trace)")
     ap.add_argument("--summarize-trace", nargs=2, metavar=("KERNEL_TRACE_CSV", "OUT_MD"))
     ap.add_argument("--trace-names", default="Kernel time, 3-level AMR Poisson (base 256^3, 113.5 M cells);"
                     "FP64 solve (timed);mixed-precision solve (timed)")
@@ -704,7 +713,7 @@ def main():
     if not args.no_tune:
         t0 = time.time()
         tune = solver.tune_relax()
-        log(f"relaxation tuned in {time.time() - t0:.2f}s: " +
+        log(f"single-iteration relaxation tuned in {time.time() - t0:.2f}s: " +
             ", ".join(f"{r['kind']}{r['index']} {r['shape'][0]}x{r['shape'][1]}/kc{r['kc']} {r['ms']:.3f}ms"
                       for r in tune))
     for w in range(args.warmup):
@@ -815,8 +824,10 @@ def main():
             "launches": prof["launches"],
             "measured_copy_GBs": round(copy_gbs, 1) if copy_gbs else None,
         },
-        "relax_tiles": ({f"{r['kind']}{r['index']}": f"{r['shape'][0]}x{r['shape'][1]}/kc{r['kc']}" for r in tune}
-                        if tune else None),
+        # the tuner's picks, for single iterations only: the timed solve's relaxations come in pairs, whose
+        # launches (k_gsrb_zmarch2, k_block_visit) have tiles of their own
+        "tuned_single_iteration_tiles": ({f"{r['kind']}{r['index']}": f"{r['shape'][0]}x{r['shape'][1]}/kc{r['kc']}"
+                                          for r in tune} if tune else None),
         "mixed_precision": mixed,
         "variable_coefficients": vcout,
         "heat": heat,

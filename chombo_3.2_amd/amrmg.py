@@ -274,9 +274,11 @@ class AMRMultiGrid:
     RELAX_CHUNKS = [0, 8, 16, 32]
 
     def tune_relax(self):
-        """Autotunes the one-launch relaxation on every level that uses it; returns one
-        dict per tuned level (kind 'amr' or 'mg', index, cells, chosen shape and
-        z-chunk, ms per iteration, all timings [shape][chunk])."""
+        """Autotunes the one-launch relaxation on every level that uses it, for later single
+        iterations (pairs of iterations and the visits of levels of up to a million cells
+        run in kernels of their own, which are not tuned); returns one dict per tuned level
+        (kind 'amr' or 'mg', index, cells, chosen shape and z-chunk, ms per iteration, all
+        timings [shape][chunk])."""
         cap = 64
         w = 6 + len(self.RELAX_SHAPES) * len(self.RELAX_CHUNKS)
         tab = np.zeros(cap * w)
