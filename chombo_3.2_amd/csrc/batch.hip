@@ -252,8 +252,9 @@ __global__ void k_batch_zero_norms(double* norms, const int* active, int n) {
 }
 
 // ---------------------------------------------------------------------------
-// The general bottom kernel, for levels whose slot tables do not apply (bottom.hip): relax(m_bottom) from zero, then BiCGStabSolver::solve
-// (BiCGStabSolver.H:199-519) in FP64 on the deepest level, one workgroup per problem.
+// The general bottom kernel, for levels whose slot tables do not apply (bottom.hip):
+// relax(m_bottom) from zero, then BiCGStabSolver::solve (BiCGStabSolver.H:199-519) in FP64 on the
+// deepest level, one workgroup per problem.
 // Level operations mirror AMRPoissonOp on that level (homogeneous BC) and the
 // reductions keep the reference orders (dot: per box serially in Fortran order,
 // boxes in layout order; norm 2: FArrayBox::sumPow column sums per box).
@@ -1111,9 +1112,11 @@ BatchSolver::BatchSolver(Context* ctx, std::vector<BatchProblemSpec> problems, i
   d_resPtr = (void**)upload(m_ctx, resp, &m_bytes);
   d_bscratchOff = upload(m_ctx, h_bscratchOff, &m_bytes);
   alloc((void**)&d_bscratch, sizeof(double) * soff);
-  // every depth starts with the tile shape of its largest problem's size, its chunks by the
-  // work of all (96 problems of 16^3 to 128^3, FP32, three lanes: 55.9 ms with the former 64 x 8
-  // columns and 55.7 ms, another lane's bottoms bound it; one 64^3 relaxation 11.2 and 6.2 us)
+  // every depth starts with the tile shape of its largest problem's size, its chunks by the work of
+  // all.  Whole solves, milliseconds, with 64 x 8 columns everywhere and so (FP64 / mixed): 64
+  // problems of 32^3 4.14 -> 3.02 / 3.50 -> 2.57, 16 of 64^3 4.90 -> 3.85 / 4.17 -> 3.26, 4 of 128^3 6.78 ->
+  // 6.01 / 5.79 -> 4.95, 48 of 16^3 to 48^3 5.41 -> 4.44 / 4.86 -> 4.11; 96 of 16^3 to 128^3, which
+  // bottoms bound, 67.5 -> 64.2 / 62.1 -> 59.3, in three lanes 56.4 -> 54.7 / 53.0 -> 52.2
   for (int d = 0; d < D; d++) {
     const Depth& L = m_depth[d];
     long long most = 0;

@@ -1,6 +1,6 @@
 // A smoothing visit of a small merged level in one launch.
 //
-// What bounds it: on levels of up to a few million cells the V-cycle is a chain of launches, each
+// What bounds it: on levels of up to about a million cells the V-cycle is a chain of launches, each
 // a few microseconds of dependent latency (a z march of six planes takes 6.5 us however small
 // the level), with all data in L2.  So a workgroup takes a block of BX x BY x BZ cells with a halo
 // wide enough for the whole visit into LDS in one go, all loads in flight together, and runs

@@ -583,7 +583,8 @@ __global__ void __launch_bounds__(NT) k_bottom(BottomLaunch<T> A) {
     for (m = 2 * m; m < n; m++) acc += st[m];
     return acc;
   };
-  // the terms st[0], st[stride], ... of a box column (at most a few hundred)
+  // the terms st[0], st[stride], ... of a box column's rows in this stage: as many as LDS holds, serially
+  // in one thread (a box of 2 x 90 x 90 cells has 8100 rows in one stage, and two threads add them)
   auto column_sum = [&](const double* st, int n, int stride, double acc, bool assign) {
     constexpr int K = 4;
     if (assign && n > 0) {
@@ -623,8 +624,8 @@ __global__ void __launch_bounds__(NT) k_bottom(BottomLaunch<T> A) {
             cell(x.c.y, x.u.b, x.w.b);
           });
   };
-  // Tree order: each thread adds its entries' terms (red, then black), then a fixed pairwise
-  // tree over the 1024 threads; the result depends only on the level
+  // Tree order: each thread adds its entries' terms (red, then black), the 64 threads of a wave are
+  // added pairwise, and the 16 waves' sums in order; the result depends only on the level
   auto tree_sum = [&](const D2* a1, const D2* b1) {
     double acc = 0.0;
     each([&](int i) {

@@ -634,10 +634,11 @@ int amrmg_bottom_solve_device(amrmg_solver* s, double* corr, const double* res, 
   DeviceBottomSolver<double> b(s->ctx->c.get());
   copy_bottom_params(b.m_fallback, s->bottom->m_fallback);
   b.define(op, true);
-  // (this entry point takes one array of at most 256 boxes and 512 box columns)
+  // (this entry point's own limits, see amrmg.h; a solve's bottom has none of them)
   long long widths = 0;
   for (const Box& x : L->dbl.boxes) widths += x.len(0);
-  if (!b.onDevice() || !L->merged || 2 * L->nbox > 512 || widths > 512) throw std::runtime_error("the deepest multigrid level does not allow the device bottom solver");
+  if (!b.onDevice() || !L->merged || 2 * L->nbox > 512 || widths > 512)
+    throw std::runtime_error("the deepest multigrid level does not allow the device bottom solver");
   LevelData<double> c(L), r(L);
   upload_valid(*L, c.d, corr);
   upload_valid(*L, r.d, res);

@@ -69,7 +69,7 @@ __device__ __forceinline__ void vc_zmarch_body(const ops::FusedArgs& a, const VC
   const int nx = a.hi[0] - a.lo[0] + 1;
   const int d1 = min(di + 1, nx - 1) - di, d2 = min(di + 2, nx) - di;  // second cell and third x face
   // a lane's place in a plane in bytes: with the plane's address uniform, each access is a scalar
-  // base and a 32-bit offset (the launcher checks that a plane has less than 2^32 bytes)
+  // base and a 32-bit offset (the launcher takes this march only where a plane has less than 2^31 bytes)
   const unsigned oc = (unsigned)(di + 1 + (dj + 1) * a.sy) * (unsigned)sizeof(T);
   const unsigned of0 = (unsigned)(di + dj * vc.fsy[0]) * (unsigned)sizeof(T), of02 = of0 + d2 * (unsigned)sizeof(T);
   const unsigned of1 = (unsigned)(di + dj * vc.fsy[1]) * (unsigned)sizeof(T), of11 = of1 + d1 * (unsigned)sizeof(T);

@@ -177,8 +177,11 @@ int amrmg_average(amrmg_solver* s, int lev, const double* fine, double* coarse);
 int amrmg_bottom_solve(amrmg_solver* s, double* corr, const double* res, int nbottom, double metric, double eps,
                        int* info);
 /* The same on the device bottom solver the solves use (one workgroup, no host round
-   trip per iteration; the deepest multigrid level must be stored as one array over
-   its whole domain, with constant coefficients); info = {iterations} */
+   trip per iteration).  This entry point takes one-component fields on a level stored as one
+   array over its whole domain (no periodic or quadratic faces), of constant coefficients, with
+   at most 256 boxes and at most 512 box columns in all (the sum of the boxes' x extents), and
+   refuses others; a solve's own bottom also takes per-box and periodic levels and several
+   components.  info = {iterations} */
 int amrmg_bottom_solve_device(amrmg_solver* s, double* corr, const double* res, int nbottom, double metric,
                               double eps, int* info);
 /* BiCGStabSolver's public parameters (BiCGStabSolver.H:105-153) for every bottom solve of
